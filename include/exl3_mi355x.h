@@ -232,6 +232,23 @@ int exl3_prefill_matmul(const uint16_t* xh, const uint16_t* w_t, int rows, int k
  * entry point then rejects). */
 size_t exl3_prefill_matmul_workspace_bytes(int rows, int k, int n);
 
+/* Prefill contraction for few rows: the same product as exl3_prefill_gemm / exl3_prefill_matmul, each weight decoded
+ * from the trellis straight into MFMA operand registers (no fp16 weights in memory), up to 256 rows per decode. The
+ * form for short prompts, prompt chunks and decode batches, where reconstructing the weights costs more than the
+ * product; replaces decode_wt + matmul + hadamard_transform + svh of linear.py:97-105.
+ *   xh fp16 (rows, k) (already rotated), 16-byte aligned; trellis as in exl3_gemv; svh fp16 [n]; bias NULL or [n] in
+ *   out_dtype (added after the rounding to out_dtype and rounded again); y (rows, n) in out_dtype, 16-byte aligned.
+ *   k % 64 == 0, n % 128 == 0, 1 <= rows <= 65535; activations, trellis and rows x n x 4 bytes each below 2 GiB.
+ *   splits: workgroups per (row block, column block) over k, 0 = automatic; more than one needs a 16-byte aligned
+ *   workspace of exl3_prefill_rows_workspace_bytes(rows, k, n, K, splits) bytes (uninitialised is fine) and a second
+ *   launch that adds the splits' fp32 sums in order. Deterministic; the split depends on the shape only. */
+int exl3_prefill_rows(const uint16_t* xh, const uint32_t* trellis, int k, int n, int K, int cb, const uint16_t* svh,
+                      const void* bias, void* y, int out_dtype, int rows, int splits, void* workspace,
+                      size_t workspace_bytes, void* stream);
+
+/* Workspace bytes exl3_prefill_rows needs (0: none; also 0 for an invalid shape, which the entry point rejects). */
+size_t exl3_prefill_rows_workspace_bytes(int rows, int k, int n, int K, int splits);
+
 /* Output rotation for a prefill whose GEMM runs elsewhere (bench.py's platform-BLAS comparison, built as
  * the reference's prefill is, linear.py:97-105): exl3_reconstruct writes W_inner^T (bit-exact fp16), the
  * caller multiplies g = xh @ W_inner in fp16 with fp32 accumulation using its BLAS library, and this entry

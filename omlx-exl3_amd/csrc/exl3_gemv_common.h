@@ -47,6 +47,14 @@ constexpr int kBufferFlags = 0x00020000;   // raw buffer descriptor word 3 (32-b
 //   pair : b[p/2] = (w_p, w_{p+1}) fp16, p even, 16 registers
 // The hash is the 32-bit multiply form (window_clean + hash32); exl3_codebook checks it against the 16-bit form
 // for every state.
+// decode_pair: register I of the pair form, the fp16-rounded values of positions 2 I and 2 I + 1.
+template <int K, int CB, int I>
+__device__ __forceinline__ uint32_t decode_pair(const uint32_t* w, uint32_t wp, uint32_t xor_v) {
+  const uint32_t h0 = hash32<CB>(window_clean<K, 2 * I>(w, wp)), h1 = hash32<CB>(window_clean<K, 2 * I + 1>(w, wp));
+  if constexpr (CB == 2) return mul1_pair(mul1_r(h0), mul1_r(h1));
+  else return values2_h(h0, h1, kMask3, xor_v);
+}
+
 template <int K, int CB, bool SPLIT>
 __device__ __forceinline__ void decode_run(const uint32_t* w, uint32_t wp, uint32_t* b, uint32_t xor_v) {
   if constexpr (SPLIT) {
@@ -55,16 +63,10 @@ __device__ __forceinline__ void decode_run(const uint32_t* w, uint32_t wp, uint3
       summands2_h(hash32<CB>(window_clean<K, p>(w, wp)), hash32<CB>(window_clean<K, p + 1>(w, wp)), kMask3, xor_v,
                   b[p], b[p + 1]);
     });
-  } else if constexpr (CB == 2) {
-    static_for<0, 16>([&](auto P) {
-      constexpr int p = 2 * decltype(P)::value;
-      b[p / 2] = mul1_pair(mul1_r(hash32<CB>(window_clean<K, p>(w, wp))), mul1_r(hash32<CB>(window_clean<K, p + 1>(w, wp))));
-    });
   } else {
     static_for<0, 16>([&](auto P) {
-      constexpr int p = 2 * decltype(P)::value;
-      b[p / 2] = values2_h(hash32<CB>(window_clean<K, p>(w, wp)), hash32<CB>(window_clean<K, p + 1>(w, wp)), kMask3,
-                           xor_v);
+      constexpr int i = decltype(P)::value;
+      b[i] = decode_pair<K, CB, i>(w, wp, xor_v);
     });
   }
 }

@@ -20,6 +20,7 @@
 #include "exl3_capi_common.h"
 #include "exl3_device.h"
 #include "exl3_gemv_common.h"
+#include "exl3_prefill_reduce.h"
 
 namespace exl3 {
 
@@ -446,16 +447,26 @@ __global__ __launch_bounds__(256) void prefill_mm_reduce_kernel(const float* __r
   const int lane = threadIdx.x & 63;
   const int c0 = b * 128 + 8 * (lane & 15);
   const size_t o0 = (size_t)r * n + c0, split = (size_t)rows * n, oy = (size_t)r * ldy + c0;
-  float e[8];
-  {
-    const f32x4* p = reinterpret_cast<const f32x4*>(partials + o0);
-    const f32x4 a = p[0], bb = p[1];
-    e[0] = a.x; e[1] = a.y; e[2] = a.z; e[3] = a.w; e[4] = bb.x; e[5] = bb.y; e[6] = bb.z; e[7] = bb.w;
-  }
-  for (int s = 1; s < S; ++s) {
-    const f32x4* p = reinterpret_cast<const f32x4*>(partials + s * split + o0);
-    const f32x4 a = p[0], bb = p[1];
-    e[0] += a.x; e[1] += a.y; e[2] += a.z; e[3] += a.w; e[4] += bb.x; e[5] += bb.y; e[6] += bb.z; e[7] += bb.w;
+  // the splits in order, four splits' loads in flight at a time (a slot past S re-reads split S - 1, unused)
+  float e[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int s0 = 0; s0 < S; s0 += 4) {
+    f32x4 t[4][2];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const f32x4* p = reinterpret_cast<const f32x4*>(partials + (size_t)min(s0 + u, S - 1) * split + o0);
+      t[u][0] = p[0];
+      t[u][1] = p[1];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if (s0 + u < S) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          e[i] += t[u][0][i];
+          e[4 + i] += t[u][1][i];
+        }
+      }
+    }
   }
   fwht128_lane8(e, lane);
   float o[8];
@@ -463,8 +474,16 @@ __global__ __launch_bounds__(256) void prefill_mm_reduce_kernel(const float* __r
   for (int i = 0; i < 8; ++i) {
     o[i] = round_through<OT>(e[i] * kHadScale * f16_to_f32(svh[c0 + i]));
     if (bias) o[i] = round_through<OT>(o[i] + load_as_f32<OT>(bias, c0 + i));
-    store_from_f32<OT>(y, oy + i, o[i]);
   }
+  store8<OT>(y, oy, o);
+}
+
+void launch_prefill_reduce(const float* partials, int S, int rows, int n, const uint16_t* svh, const void* bias,
+                           void* y, int ldy, int out_dtype, hipStream_t st) {
+  const int groups = rows * (n / 128), grid = (groups + 15) / 16;
+  if (out_dtype == kF16) prefill_mm_reduce_kernel<kF16><<<grid, 256, 0, st>>>(partials, S, rows, n, groups, svh, bias, y, ldy);
+  else if (out_dtype == kBF16) prefill_mm_reduce_kernel<kBF16><<<grid, 256, 0, st>>>(partials, S, rows, n, groups, svh, bias, y, ldy);
+  else prefill_mm_reduce_kernel<kF32><<<grid, 256, 0, st>>>(partials, S, rows, n, groups, svh, bias, y, ldy);
 }
 
 template <int OT, int TI>
@@ -481,11 +500,7 @@ static void launch_mm(const MmPlan& p, const uint16_t* xh, const uint16_t* wt, i
   if (p.ti == 4) launch_mm_ti<OT, 4>(p, xh, wt, rows, k, n, svh, bias, y, ldy, partials, st);
   else if (p.ti == 3) launch_mm_ti<OT, 3>(p, xh, wt, rows, k, n, svh, bias, y, ldy, partials, st);
   else launch_mm_ti<OT, 2>(p, xh, wt, rows, k, n, svh, bias, y, ldy, partials, st);
-  if (p.splits > 1) {
-    const int groups = rows * (n / 128);
-    prefill_mm_reduce_kernel<OT><<<(groups + 15) / 16, 256, 0, st>>>(partials, p.splits, rows, n, groups, svh, bias,
-                                                                     y, ldy);
-  }
+  if (p.splits > 1) launch_prefill_reduce(partials, p.splits, rows, n, svh, bias, y, ldy, OT, st);
 }
 
 }  // namespace exl3

@@ -1,0 +1,11 @@
+// SPDX-License-Identifier: Apache-2.0
+// Few-row prefill kernels of the MCG codebook.
+#include "exl3_prefill_rows_body.h"
+
+namespace exl3 {
+
+void rows_launch_cb1(int K, int rt, const dim3& grid, const RowsArgs& a, hipStream_t st) {
+  launch_rows_k<1>(K, rt, grid, a, st);
+}
+
+}  // namespace exl3

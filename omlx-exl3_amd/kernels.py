@@ -1,9 +1,9 @@
 # SPDX-License-Identifier: Apache-2.0
 """Host-side wrappers of the HIP kernels, mirroring the reference's kernel API
 (src/omlx/exl3/kernels.py): decode_wt, rot, norm_rot, swiglu_rot, TrellisGemvPlan, MAX_GEMV_ROWS, plus
-prefill_gemm (the replacement of decode_wt + matmul + Hadamard on the prefill path: weights reconstructed
-in bounded column windows, each multiplied by a hand-written MFMA GEMM with the output rotation in its
-epilogue, or one fused launch) and codebook (the codebook diagnostic).
+prefill_gemm (the replacement of decode_wt + matmul + Hadamard on the prefill path: weights decoded into MFMA
+operands for few rows, else reconstructed in bounded column windows, each multiplied by a hand-written MFMA GEMM
+with the output rotation in its epilogue, or one fused launch) and codebook (the codebook diagnostic).
 
 Tensors are torch tensors on the HIP device; every call is enqueued on torch's current stream and returns
 without synchronising. Argument errors raise before anything is launched (the reference asserts,
@@ -338,6 +338,27 @@ def prefill_matmul(xh: torch.Tensor, wt: torch.Tensor, svh: torch.Tensor, bias: 
     return out
 
 
+def prefill_rows(xh: torch.Tensor, trellis: torch.Tensor, k: int, n: int, K: int, cb: int, svh: torch.Tensor,
+                 bias: torch.Tensor | None, out: torch.Tensor, splits: int = 0) -> torch.Tensor:
+    """had128(xh @ W_inner) * svh (+ bias) into out (rows, n) for few rows: each weight decoded from the trellis into
+    MFMA operand registers, no fp16 weights in memory (exl3_prefill_rows). k is split over workgroups (`splits`,
+    0 = automatic); the splits' fp32 workspace is allocated here, from PyTorch's caching allocator, for the call."""
+    _dev(xh, "xh")
+    _dev(out, "out")
+    rows = xh.numel() // k
+    _require(xh.dtype == torch.float16 and xh.numel() == rows * k, "xh must be fp16 (rows, k)")
+    _require(out.numel() == rows * n and out.dtype in DTYPE_CODE, "prefill_rows: out must be (rows, n) fp16/bf16/fp32")
+    trellis_words(trellis, k, n, K)
+    _check_vec(svh, n, torch.float16, "svh")
+    _check_vec(bias, n, out.dtype, "bias")
+    nbytes = lib().exl3_prefill_rows_workspace_bytes(rows, k, n, K, splits)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=xh.device) if nbytes else None
+    check(lib().exl3_prefill_rows(ptr(xh), ptr(trellis), k, n, K, cb, ptr(svh), ptr(bias), ptr(out),
+                                  DTYPE_CODE[out.dtype], rows, splits, ptr(ws), nbytes, stream_handle(xh.device)),
+          "exl3_prefill_rows")
+    return out
+
+
 def prefill_out_rotate(g: torch.Tensor, svh: torch.Tensor, bias: torch.Tensor | None,
                        out: torch.Tensor) -> torch.Tensor:
     """The output rotation of a prefill product g = xh @ W_inner (rows, n) fp16 computed by some other GEMM:
@@ -378,17 +399,29 @@ def prefill_chunks(n: int, k: int, chunk_bytes: int = PREFILL_CHUNK_BYTES) -> li
 PREFILL_PATHS = ("auto", "matmul", "fused")
 
 
+def takes_rows_form(rows: int, k: int, n: int, K: int) -> bool:
+    """Whether prefill_gemm's "auto" decodes the weights into MFMA operands (prefill_rows) instead of reconstructing
+    them first. Measured on MI355X (us, prefill_rows / reconstruction + GEMM): 5120 -> 17408 at 33 / 512 / 640 / 777 /
+    1000 rows 26 / 115 / 139 / 175 / 229 against 77 / 136 / 156 / 186 / 220; 1024 -> 8192 at 640 / 1000 rows 25 / 31
+    against 31 / 33; 4096 -> 4096 at 640 / 1000 rows 39 / 57 against 42 / 54. Narrow outputs of a long k, whose GEMM has
+    few tiles, stay ahead to about 1,000 rows: 17408 -> 5120 at 777 / 1000 rows 178 / 196 against 192 / 205 (with k split
+    for the GEMM too), 5120 -> 1024 at 1000 rows 28 against 30. The size limits are the entry point's."""
+    return (rows <= 640 or rows <= 1024 and k >= 2 * n) and k % 64 == 0 and n % 128 == 0 and \
+        max(2 * rows * k, 4 * rows * n, (k + 128) * n * K // 8) < 1 << 31
+
+
 def prefill_gemm(xh: torch.Tensor, trellis: torch.Tensor, k: int, n: int, K: int, cb: int, svh: torch.Tensor,
                  bias: torch.Tensor | None = None, out_dtype: torch.dtype = torch.float16,
                  out: torch.Tensor | None = None, path: str = "auto",
                  chunk_bytes: int = PREFILL_CHUNK_BYTES) -> torch.Tensor:
     """had128(xh @ W_inner) * svh (+ bias) for xh (rows, k) fp16 (already rotated) (linear.py:97-105).
-    path "matmul": W_inner^T reconstructed (exl3_reconstruct, bit-exact fp16) one column window at a time
+    path "auto": weights decoded into MFMA operands for few rows (prefill_rows, by the rule of takes_rows_form), else
+    "matmul" (k a multiple of 64, as every EXL3 layer's is), else "fused"; "matmul": W_inner^T reconstructed
+    (exl3_reconstruct, bit-exact fp16) one column window at a time
     (prefill_chunks: at most chunk_bytes of fp16 weights alive, one buffer reused), each window multiplied by the
     hand-written MFMA GEMM with the output rotation in its epilogue (exl3_prefill_matmul, writing its columns of
     the output in place; k split over workgroups for few rows); "fused": weights reconstructed in LDS and
-    contracted on MFMA in one launch (exl3_prefill_gemm); "auto": "matmul" (k a multiple of 64, as every EXL3
-    layer's is), else "fused"."""
+    contracted on MFMA in one launch (exl3_prefill_gemm)."""
     _dev(xh, "xh")
     rows = xh.numel() // k
     _require(xh.dtype == torch.float16 and xh.numel() == rows * k, "xh must be fp16 (rows, k)")
@@ -403,10 +436,13 @@ def prefill_gemm(xh: torch.Tensor, trellis: torch.Tensor, k: int, n: int, K: int
     else:
         _check_out(out, (rows, n), out_dtype)
         _require(not _overlap(out, xh), "prefill_gemm: out must not overlap xh")
+    rows_form = path == "auto" and takes_rows_form(rows, k, n, K)
     if path == "auto":
         path = "matmul" if k % 64 == 0 else "fused"
     if path == "matmul":
-        chunks = prefill_chunks(n, k, chunk_bytes)
+        chunks = prefill_chunks(n, k, chunk_bytes)     # (also the rows form's check of the caller's bound)
+        if rows_form:
+            return prefill_rows(xh, trellis, k, n, K, cb, svh, bias, out)
         x2 = xh.reshape(rows, k).contiguous()
         y2 = out.view(rows, n)
         wt = torch.empty((chunks[0][1], k), dtype=torch.float16, device=xh.device)
@@ -452,5 +488,5 @@ def attn_decode_rotate(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cach
 
 
 __all__ = ["MAX_GEMV_ROWS", "GEMV_ROWS_LIMIT", "TrellisGemvPlan", "decode_wt", "rot", "norm_rot", "swiglu_rot",
-           "prefill_gemm", "prefill_chunks", "prefill_matmul", "prefill_out_rotate", "PREFILL_CHUNK_BYTES", "codebook",
+           "prefill_gemm", "prefill_chunks", "prefill_matmul", "prefill_rows", "takes_rows_form", "prefill_out_rotate", "PREFILL_CHUNK_BYTES", "codebook",
            "attn_decode_rotate", "Exl3Error"]

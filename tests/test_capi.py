@@ -252,3 +252,28 @@ def test_package_fails_loudly_without_library(tmp_path, monkeypatch):
     monkeypatch.setattr(_capi, "_lib", None)
     with pytest.raises(_capi.Exl3Error):
         _capi.lib()
+
+
+def test_prefill_rows_argument_errors(capi):
+    """Host-side checks of the few-row prefill and its workspace query (the pointers are never dereferenced)."""
+    lib = capi.lib()
+    p = ctypes.c_void_p(0x10000)
+
+    def rows_(xh=p, tr=p, k=512, n=256, K=6, cb=0, svh=p, y=p, ot=0, rows=9, splits=2, ws=None, wsb=0):
+        return lib.exl3_prefill_rows(xh, tr, k, n, K, cb, svh, None, y, ot, rows, splits, ws, wsb, None)
+
+    assert rows_(xh=None) == -1 and "NULL" in _err(capi)
+    assert rows_(k=96) == -1 and "multiple of 64" in _err(capi)
+    assert rows_(n=192) == -1 and "multiple of 128" in _err(capi)
+    assert rows_(K=9) == -1 and "K must be" in _err(capi)
+    assert rows_(cb=3) == -1 and "codebook" in _err(capi)
+    assert rows_(rows=0) == -1 and "rows" in _err(capi)
+    assert rows_(rows=65536) == -1 and "rows" in _err(capi)
+    assert rows_(ot=3) == -1 and "out_dtype" in _err(capi)
+    assert rows_(xh=ctypes.c_void_p(0x10008)) == -1 and "aligned" in _err(capi)
+    assert rows_(k=1 << 16, n=1 << 17) == -1 and "2 GiB" in _err(capi)
+    assert rows_() == -2 and "workspace" in _err(capi)
+    assert lib.exl3_prefill_rows_workspace_bytes(9, 512, 256, 6, 2) == 2 * 9 * 256 * 4
+    assert lib.exl3_prefill_rows_workspace_bytes(9, 512, 256, 6, 1) == 0
+    assert lib.exl3_prefill_rows_workspace_bytes(9, 512, 256, 6, 100) == 8 * 9 * 256 * 4   # one step per split at most
+    assert lib.exl3_prefill_rows_workspace_bytes(9, 500, 256, 6, 2) == 0                   # invalid shape
