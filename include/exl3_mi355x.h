@@ -278,6 +278,24 @@ int exl3_attn_decode_rotate(const uint16_t* q, const uint16_t* k, const uint16_t
                             int n_heads, int n_kv_heads, int head_dim, int max_len, const uint16_t* suh,
                             uint16_t* o, uint16_t* xh, void* stream);
 
+/* exl3_attn_decode_rotate with a workspace: the positions are spread over workgroups, each serving a group of a
+ * key/value head's query heads (a cached row is read once per group), and their results merged.
+ *   workspace  exl3_attn_decode_workspace_bytes(n_heads, n_kv_heads, max_len) bytes, 16-byte aligned, uninitialised is
+ *              fine, not shared by calls in flight together; NULL runs exl3_attn_decode_rotate
+ *   counters   NULL: a second launch merges; or n_heads x 256 bytes (uint32 every 64 words) zeroed once before the first
+ *              use, with the workspace's rules: the last workgroup to arrive merges, in the one launch, and leaves the
+ *              counters at zero (the faster form up to a max_len of about 2,048)
+ * Other arguments, cache writes and rounding points as exl3_attn_decode_rotate; the sums over positions are added in
+ * another order (fixed by the position and the shape: results are reproducible). */
+int exl3_attn_decode_rotate_ws(const uint16_t* q, const uint16_t* k, const uint16_t* v, uint16_t* k_cache,
+                               uint16_t* v_cache, const int64_t* pos, const float* rope_cos, const float* rope_sin,
+                               int n_heads, int n_kv_heads, int head_dim, int max_len, const uint16_t* suh,
+                               uint16_t* o, uint16_t* xh, void* workspace, size_t workspace_bytes, uint32_t* counters,
+                               void* stream);
+
+/* Workspace bytes of exl3_attn_decode_rotate_ws (0: invalid sizes, which the entry point rejects). */
+size_t exl3_attn_decode_workspace_bytes(int n_heads, int n_kv_heads, int max_len);
+
 #ifdef __cplusplus
 }
 #endif

@@ -457,12 +457,31 @@ def prefill_gemm(xh: torch.Tensor, trellis: torch.Tensor, k: int, n: int, K: int
     return out
 
 
+# Decode attention by cache capacity: one workgroup per head up to the first bound; above it the positions are split
+# over workgroups, merged by the last to arrive up to the second bound when the caller holds an attn_workspace, else by
+# a second launch (exl3_attn_decode_rotate_ws; measured sides at csrc/exl3_attn.hip's plan).
+ATTN_UNSPLIT_LEN = 512
+ATTN_WORKSPACE_LEN = 2048
+ATTN_MAX_LEN = 8192
+
+
+def attn_workspace(n_heads: int, n_kv: int, max_len: int, device) -> torch.Tensor | None:
+    """A zeroed workspace for attn_decode_rotate calls of this shape that follow each other on one stream (arrival
+    counters, left at zero by every call, and the workgroups' sums), or None for a capacity that takes none."""
+    if not ATTN_UNSPLIT_LEN < max_len <= ATTN_WORKSPACE_LEN:
+        return None
+    nbytes = lib().exl3_attn_decode_workspace_bytes(n_heads, n_kv, max_len)
+    _require(nbytes > 0, "attn_workspace: bad head counts")
+    return torch.zeros(256 * n_heads + nbytes, dtype=torch.uint8, device=device)
+
+
 def attn_decode_rotate(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor,
                        v_cache: torch.Tensor, pos: torch.Tensor, rope_cos: torch.Tensor, rope_sin: torch.Tensor,
-                       suh: torch.Tensor | None, want_o: bool = False):
+                       suh: torch.Tensor | None, want_o: bool = False, workspace: torch.Tensor | None = None):
     """Batch-1 decode attention with rotary embedding and KV-cache append, producing o_proj's rotated input
     (exl3_attn_decode_rotate). q (n_heads*128,), k / v (n_kv*128,) fp16 (views of one row are fine);
     caches fp16 (n_kv, max_len, 128); pos int64 (1,) on the device; rope tables fp32 (max_len, 64).
+    workspace: attn_workspace of this shape, held by the caller, or None (one is allocated where it is needed).
     Returns (xh (1, 1, n_heads*128) or None, o (1, n_heads*128) or None)."""
     for t, name in ((k_cache, "k_cache"), (v_cache, "v_cache"), (rope_cos, "rope_cos"), (rope_sin, "rope_sin")):
         _dev(t, name)
@@ -481,12 +500,26 @@ def attn_decode_rotate(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cach
     if suh is not None:
         _require(suh.dtype == torch.float16 and suh.numel() == n_heads * hd and suh.is_contiguous(),
                  "attn_decode_rotate: suh fp16 (n_heads*128,)")
-    check(lib().exl3_attn_decode_rotate(ptr(q), ptr(k), ptr(v), ptr(k_cache), ptr(v_cache), ptr(pos), ptr(rope_cos),
-                                        ptr(rope_sin), n_heads, n_kv, hd, max_len, ptr(suh), ptr(o), ptr(xh),
-                                        stream_handle(q.device)), "exl3_attn_decode_rotate")
+    args = (ptr(q), ptr(k), ptr(v), ptr(k_cache), ptr(v_cache), ptr(pos), ptr(rope_cos), ptr(rope_sin), n_heads, n_kv,
+            hd, max_len, ptr(suh), ptr(o), ptr(xh))
+    if max_len <= ATTN_UNSPLIT_LEN or max_len > ATTN_MAX_LEN:      # (the entry point refuses what is too long)
+        check(lib().exl3_attn_decode_rotate(*args, stream_handle(q.device)), "exl3_attn_decode_rotate")
+        return xh, o
+    nbytes = lib().exl3_attn_decode_workspace_bytes(n_heads, n_kv, max_len)
+    if workspace is not None and max_len <= ATTN_WORKSPACE_LEN:
+        _dev(workspace, "workspace")
+        _require(workspace.dtype == torch.uint8 and workspace.numel() == 256 * n_heads + nbytes,
+                 "attn_decode_rotate: workspace is attn_workspace of this shape")
+        counters = workspace.data_ptr()
+        ws = counters + 256 * n_heads
+    else:
+        buf = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+        counters, ws = None, buf.data_ptr()
+    check(lib().exl3_attn_decode_rotate_ws(*args, ws, nbytes, counters, stream_handle(q.device)),
+          "exl3_attn_decode_rotate")
     return xh, o
 
 
 __all__ = ["MAX_GEMV_ROWS", "GEMV_ROWS_LIMIT", "TrellisGemvPlan", "decode_wt", "rot", "norm_rot", "swiglu_rot",
            "prefill_gemm", "prefill_chunks", "prefill_matmul", "prefill_rows", "takes_rows_form", "prefill_out_rotate", "PREFILL_CHUNK_BYTES", "codebook",
-           "attn_decode_rotate", "Exl3Error"]
+           "attn_decode_rotate", "attn_workspace", "Exl3Error"]

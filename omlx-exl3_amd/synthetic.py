@@ -32,7 +32,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from .fusion import fuse_decode
-from .kernels import attn_decode_rotate
+from .kernels import attn_decode_rotate, attn_workspace
 from .linear import EXL3Linear
 from .loader import group_siblings
 
@@ -130,6 +130,9 @@ class Attention(nn.Module):
                                                     dtype=torch.float16, device=device), persistent=False)
         self.register_buffer("v_cache", torch.zeros(cfg.n_kv_heads, cfg.max_len, cfg.head_dim,
                                                     dtype=torch.float16, device=device), persistent=False)
+        split = torch.device(device).type == "cuda" and cfg.head_dim == 128      # decode attention's merge workspace
+        self.register_buffer("attn_ws", attn_workspace(cfg.n_heads, cfg.n_kv_heads, cfg.max_len, device) if split
+                             else None, persistent=False)
 
     def forward(self, x, pos, cos, sin, cos_half=None, sin_half=None):
         """x (T, hidden) fp16 at positions pos (T,) int64 (device). Decode (T = 1) attends over the cache
@@ -140,7 +143,7 @@ class Attention(nn.Module):
         nh, nkv, hd = cfg.n_heads, cfg.n_kv_heads, cfg.head_dim
         if T == 1 and self.fused_attn and cos_half is not None:
             xh, _ = attn_decode_rotate(q.reshape(-1), k.reshape(-1), v.reshape(-1), self.k_cache, self.v_cache, pos,
-                                       cos_half, sin_half, self.o_proj.rot_suh.reshape(-1))
+                                       cos_half, sin_half, self.o_proj.rot_suh.reshape(-1), workspace=self.attn_ws)
             return self.o_proj.gemv_rotated(xh, x.dtype, self.o_proj._bias_for(x.dtype))
         c, s = cos[pos].unsqueeze(1), sin[pos].unsqueeze(1)                       # (T, 1, hd)
         q = q.view(T, nh, hd).float()
