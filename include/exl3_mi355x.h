@@ -218,9 +218,9 @@ int exl3_prefill_gemm(const uint16_t* xh, const uint32_t* trellis, int k, int n,
  *   out_dtype with a row stride of ldy elements (ldy >= n; ldy times the element size a multiple of 16 bytes),
  *   16-byte aligned, so a column chunk of a wider output writes its slice in place.
  *   k % 64 == 0, n % 128 == 0, rows >= 1; xh and w_t each below 2 GiB.
- *   When the shape's tiles would leave at least half of the GPU's CUs idle (few rows), k is split over several
- *   workgroups per tile and a second launch adds the splits in a fixed order: that needs a 16-byte aligned
- *   workspace of exl3_prefill_matmul_workspace_bytes(rows, k, n) bytes (0 when no split is made: the workspace
+ *   Where the shape's tiles alone would leave CUs idle (few rows, narrow outputs), k is split over several workgroups
+ *   per tile and a second launch adds the splits in a fixed order: that needs a 16-byte aligned workspace of
+ *   exl3_prefill_matmul_workspace_bytes(rows, k, n) bytes (0 when no split is made: the workspace
  *   may then be NULL); EXL3_ERR_WORKSPACE when it is missing or small. Results are deterministic; the split
  *   depends on the shape only, so a row's result can differ in the last bits between prefill calls of
  *   different row counts (the reference's MLX matmul is not row-exact either). Allocates nothing. */
@@ -231,6 +231,14 @@ int exl3_prefill_matmul(const uint16_t* xh, const uint16_t* w_t, int rows, int k
 /* Workspace bytes exl3_prefill_matmul needs for a shape (0: none; also 0 for an invalid shape, which the
  * entry point then rejects). */
 size_t exl3_prefill_matmul_workspace_bytes(int rows, int k, int n);
+
+/* exl3_prefill_matmul for a window of n columns of a call of n_call columns: tile height and k split are chosen from
+ * n_call, so a call done in windows adds each element's products in the order of the call done at once (the same bits).
+ * exl3_prefill_matmul is n_call = n. The workspace query likewise. */
+int exl3_prefill_matmul_window(const uint16_t* xh, const uint16_t* w_t, int rows, int k, int n, int n_call,
+                               const uint16_t* svh, const void* bias, void* y, int ldy, int out_dtype,
+                               void* workspace, size_t workspace_bytes, void* stream);
+size_t exl3_prefill_matmul_window_workspace_bytes(int rows, int k, int n, int n_call);
 
 /* Prefill contraction for few rows: the same product as exl3_prefill_gemm / exl3_prefill_matmul, each weight decoded
  * from the trellis straight into MFMA operand registers (no fp16 weights in memory), up to 256 rows per decode. The

@@ -42,6 +42,9 @@ _SIGNATURES = {
     "exl3_prefill_matmul": (_c_int, [_vp, _vp, _c_int, _c_int, _c_int, _vp, _vp, _vp, _c_int, _c_int, _vp, _c_size,
                                      _vp]),
     "exl3_prefill_matmul_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int]),
+    "exl3_prefill_matmul_window": (_c_int, [_vp, _vp, _c_int, _c_int, _c_int, _c_int, _vp, _vp, _vp, _c_int, _c_int,
+                                            _vp, _c_size, _vp]),
+    "exl3_prefill_matmul_window_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int]),
     "exl3_prefill_rows": (_c_int, [_vp, _vp, _c_int, _c_int, _c_int, _c_int, _vp, _vp, _vp, _c_int, _c_int, _c_int,
                                    _vp, _c_size, _vp]),
     "exl3_prefill_rows_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int, _c_int]),

@@ -375,56 +375,51 @@ __global__ __launch_bounds__(kMmThreads) __attribute__((amdgpu_waves_per_eu(2)))
   });
 }
 
-// Rows of a tile for a shape: the tiles run one per CU in rounds of 256, so the cost of a choice is its number
-// of rounds times the work of one tile (BM rows, plus a fixed part for the prologue and epilogue).
-static int mm_pick_ti(int rows, int n) {
-  const long tiles_n = (n + kMmBN - 1) / kMmBN;
-  int best = 4;
-  long best_cost = -1;
-  for (int ti = 4; ti >= 2; --ti) {
-    const long tiles = (long)((rows + 64 * ti - 1) / (64 * ti)) * tiles_n;
-    const long cost = (tiles + 255) / 256 * (64 * ti + 64);
-    if (best_cost < 0 || cost < best_cost) {
-      best = ti;
-      best_cost = cost;
-    }
-  }
-  return best;
-}
+// Launch plan of a shape (from rows, k and n only): tile height (64 ti rows) and a split of k over S workgroups per
+// tile, the pair of least estimated time. A round of w workgroups (256 at most, one per CU) takes, per 64-k step of a
+// split, a[ti] + b[ti] w / 256 us (the more CUs work, the lower the clock), and f[ti] besides; S > 1 adds the reduction
+// launch: 1.2 + 0.31 S us and S + 1 passes over an fp32 rows x n array at 3.16 TB/s (2.3 TB/s beyond 48 MB), and a
+// workspace of S x rows x n fp32, held to kMmWorkspaceLimit. At least 4 steps per split, S <= 16. The constants were
+// fitted to 111 shapes (k 1,024-17,408, n 512-17,408, 200-4,608 rows) x 3 heights x up to 8 splits, over which the pick
+// is on average within 2% of the fastest measured pair (4% for the rule before, which picked the height first and split
+// launches of at most 128 tiles). The sides, us before / now: 17408 -> 5120 at 777 / 1,024 / 1,300 rows 218 / 233 / 234
+// against 153 / 166 / 215; 5120 -> 1024 at 777 / 1,024 rows 28.5 / 33.5 against 22.9 / 24.4; 8192 -> 1024 at 3,000 rows 70
+// against 59; the largest loss, 5120 -> 1024 at 1,300 rows, 28.2 against 29.6.
+constexpr size_t kMmWorkspaceLimit = (size_t)128 << 20;
 
-// Launch plan of a shape (from rows, k and n only): tile height, and a split of k over S workgroups per tile when
-// the tiles alone would leave at least half the 256 CUs idle. S minimises an estimate of the time: rounds x steps
-// per split x ~0.55 TI us per 64-k step of a tile, plus, for S > 1, the reduction launch (S + 1 passes over an
-// fp32 rows x n array at ~4 TB/s, and ~3 us); at least 4 steps per split, at most 16 splits, the smaller S on a
-// tie. S > 1 needs a workspace of S x rows x n fp32.
 struct MmPlan {
-  int ti, tiles_m, tiles_n, splits, steps_per_split;
+  int ti, tiles_m, splits, steps_per_split;
 };
 
 static MmPlan mm_plan(int rows, int k, int n) {
-  MmPlan p;
-  p.ti = mm_pick_ti(rows, n);
-  p.tiles_m = (rows + 64 * p.ti - 1) / (64 * p.ti);
-  p.tiles_n = (n + kMmBN - 1) / kMmBN;
+  static const double a[3] = {0.575, 0.603, 0.770}, b[3] = {0.270, 0.392, 0.452}, f[3] = {3.3, 8.2, 8.9};
   const int nsteps = k / kMmBK;
-  const long tiles = (long)p.tiles_m * p.tiles_n;
-  const double step_us = 0.55 * p.ti, pass_us = (double)rows * n * 4.0 / 4.0e6;
-  int best_s = 1;
-  double best_cost = (double)((tiles + 255) / 256) * nsteps * step_us;
-  if (tiles <= 128) {
-    for (int S = 2; S <= 16; ++S) {
+  const long tiles_n = (n + kMmBN - 1) / kMmBN;
+  const double out_bytes = (double)rows * n * 4.0;
+  MmPlan best{};
+  double best_us = -1.0;
+  for (int ti = 4; ti >= 2; --ti) {
+    if (ti > 2 && rows <= 64 * (ti - 1)) continue;   // one tile row of a smaller height holds them
+    const int tiles_m = (rows + 64 * ti - 1) / (64 * ti);
+    const long tiles = (long)tiles_m * tiles_n;
+    for (int S = 1; S <= 16; ++S) {
       const int sps = (nsteps + S - 1) / S;
-      if (sps < 4) break;
-      const double cost = (double)((tiles * S + 255) / 256) * sps * step_us + (S + 1) * pass_us + 3.0;
-      if (cost < best_cost) {
-        best_s = S;
-        best_cost = cost;
+      if (S > 1 && (sps < 4 || tiles * S > 1024 || S * out_bytes > (double)kMmWorkspaceLimit)) break;
+      if ((nsteps + sps - 1) / sps != S) continue;   // an S that leaves an empty split: the plan of a smaller one
+      const long groups = tiles * S, rest = groups % 256;
+      auto round_us = [&](long w) { return sps * (a[ti - 2] + b[ti - 2] * (double)w / 256.0) + f[ti - 2]; };
+      double us = (double)(groups / 256) * round_us(256) + (rest ? round_us(rest) : 0.0);
+      if (S > 1) {
+        const double bytes = (S + 1) * out_bytes;
+        us += 1.2 + 0.31 * S + bytes / 3.16e6 + (bytes > 48e6 ? (bytes - 48e6) / 8.46e6 : 0.0);
+      }
+      if (best_us < 0 || us < best_us) {
+        best = MmPlan{ti, tiles_m, S, sps};
+        best_us = us;
       }
     }
   }
-  p.steps_per_split = (nsteps + best_s - 1) / best_s;
-  p.splits = (nsteps + p.steps_per_split - 1) / p.steps_per_split;   // no empty split
-  return p;
+  return best;
 }
 
 static size_t mm_workspace_bytes(const MmPlan& p, int rows, int n) {
@@ -489,9 +484,9 @@ void launch_prefill_reduce(const float* partials, int S, int rows, int n, const 
 template <int OT, int TI>
 static void launch_mm_ti(const MmPlan& p, const uint16_t* xh, const uint16_t* wt, int rows, int k, int n,
                          const uint16_t* svh, const void* bias, void* y, int ldy, float* partials, hipStream_t st) {
-  prefill_mm_kernel<OT, TI><<<dim3(p.tiles_m * p.tiles_n, p.splits), kMmThreads, 0, st>>>(
-      xh, wt, rows, k, n, svh, bias, y, ldy, p.tiles_m, p.tiles_n, p.splits > 1 ? partials : nullptr,
-      p.steps_per_split);
+  const int tiles_n = (n + kMmBN - 1) / kMmBN;
+  prefill_mm_kernel<OT, TI><<<dim3(p.tiles_m * tiles_n, p.splits), kMmThreads, 0, st>>>(
+      xh, wt, rows, k, n, svh, bias, y, ldy, p.tiles_m, tiles_n, p.splits > 1 ? partials : nullptr, p.steps_per_split);
 }
 
 template <int OT>
@@ -507,15 +502,26 @@ static void launch_mm(const MmPlan& p, const uint16_t* xh, const uint16_t* wt, i
 
 using namespace exl3;
 
+extern "C" size_t exl3_prefill_matmul_window_workspace_bytes(int rows, int k, int n, int n_call) {
+  if (rows < 1 || k < kMmBK || k % kMmBK != 0 || n < 128 || n % 128 != 0 || n_call < n || n_call % 128 != 0) return 0;
+  if ((uint64_t)((rows + 127) / 128) * (uint64_t)((n_call + kMmBN - 1) / kMmBN) >= (1ull << 31)) return 0;
+  return mm_workspace_bytes(mm_plan(rows, k, n_call), rows, n);
+}
+
 extern "C" size_t exl3_prefill_matmul_workspace_bytes(int rows, int k, int n) {
-  if (rows < 1 || k < kMmBK || k % kMmBK != 0 || n < 128 || n % 128 != 0) return 0;
-  if ((uint64_t)((rows + 127) / 128) * (uint64_t)((n + kMmBN - 1) / kMmBN) >= (1ull << 31)) return 0;
-  return mm_workspace_bytes(mm_plan(rows, k, n), rows, n);
+  return exl3_prefill_matmul_window_workspace_bytes(rows, k, n, n);
 }
 
 extern "C" int exl3_prefill_matmul(const uint16_t* xh, const uint16_t* w_t, int rows, int k, int n,
                                    const uint16_t* svh, const void* bias, void* y, int ldy, int out_dtype,
                                    void* workspace, size_t workspace_bytes, void* stream) {
+  return exl3_prefill_matmul_window(xh, w_t, rows, k, n, n, svh, bias, y, ldy, out_dtype, workspace, workspace_bytes,
+                                    stream);
+}
+
+extern "C" int exl3_prefill_matmul_window(const uint16_t* xh, const uint16_t* w_t, int rows, int k, int n, int n_call,
+                                          const uint16_t* svh, const void* bias, void* y, int ldy, int out_dtype,
+                                          void* workspace, size_t workspace_bytes, void* stream) {
   EXL3_REQUIRE(xh && w_t && svh && y, EXL3_ERR_ARG, "exl3_prefill_matmul: NULL pointer argument");
   EXL3_REQUIRE(k > 0 && k % kMmBK == 0, EXL3_ERR_ARG, "exl3_prefill_matmul: k must be a positive multiple of 64");
   EXL3_REQUIRE(n > 0 && n % 128 == 0, EXL3_ERR_ARG, "exl3_prefill_matmul: n must be a positive multiple of 128");
@@ -530,7 +536,11 @@ extern "C" int exl3_prefill_matmul(const uint16_t* xh, const uint16_t* w_t, int 
                EXL3_ERR_ARG, "exl3_prefill_matmul: an operand exceeds 2 GiB");
   EXL3_REQUIRE((uint64_t)((rows + 127) / 128) * (uint64_t)((n + kMmBN - 1) / kMmBN) < (1ull << 31), EXL3_ERR_ARG,
                "exl3_prefill_matmul: too many tiles");
-  const MmPlan p = mm_plan(rows, k, n);
+  EXL3_REQUIRE(n_call >= n && n_call % 128 == 0 &&
+                   (uint64_t)((rows + 127) / 128) * (uint64_t)((n_call + kMmBN - 1) / kMmBN) < (1ull << 31),
+               EXL3_ERR_ARG, "exl3_prefill_matmul_window: n_call must be a multiple of 128, at least n (%d), got %d", n,
+               n_call);
+  const MmPlan p = mm_plan(rows, k, n_call);
   const size_t need = mm_workspace_bytes(p, rows, n);
   EXL3_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && aligned(workspace, 16)), EXL3_ERR_WORKSPACE,
                "exl3_prefill_matmul: this shape splits k over %d workgroups and needs a 16-byte aligned workspace of "

@@ -314,12 +314,13 @@ class TrellisGemvPlan:
 
 
 def prefill_matmul(xh: torch.Tensor, wt: torch.Tensor, svh: torch.Tensor, bias: torch.Tensor | None,
-                   out: torch.Tensor) -> torch.Tensor:
+                   out: torch.Tensor, n_call: int | None = None) -> torch.Tensor:
     """had128(xh @ wt^T) * svh (+ bias) into out by the hand-written MFMA GEMM (exl3_prefill_matmul): xh (rows, k)
     fp16, wt (n, k) fp16 = W_inner^T (or a column window of it) as exl3_reconstruct writes it, svh / bias the n
     entries of those columns. out is (rows, n), or a column slice of a wider (rows, N) output (its row stride
-    becomes the GEMM's output stride). Shapes whose tiles would leave CUs idle split k over several workgroups;
-    their fp32 workspace is allocated here, from PyTorch's caching allocator, for the call."""
+    becomes the GEMM's output stride). n_call: the columns of the whole call when this is one window of it (the windows
+    then give the call's bits). Shapes whose tiles would leave CUs idle split k over several workgroups; their fp32
+    workspace is allocated here, from PyTorch's caching allocator, for the call."""
     k = xh.shape[-1]
     rows = xh.numel() // k
     n = wt.shape[0]
@@ -330,10 +331,11 @@ def prefill_matmul(xh: torch.Tensor, wt: torch.Tensor, svh: torch.Tensor, bias: 
     _require(out.is_cuda and out.dim() == 2 and tuple(out.shape) == (rows, n) and out.stride(1) == 1,
              "prefill_matmul: out must be (rows, n) with unit column stride")
     ldy = out.stride(0) if rows > 1 else n
-    nbytes = lib().exl3_prefill_matmul_workspace_bytes(rows, k, n)
+    n_call = n if n_call is None else n_call
+    nbytes = lib().exl3_prefill_matmul_window_workspace_bytes(rows, k, n, n_call)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=xh.device) if nbytes else None
-    check(lib().exl3_prefill_matmul(ptr(xh), ptr(wt), rows, k, n, ptr(svh), ptr(bias), ptr(out), ldy,
-                                    DTYPE_CODE[out.dtype], ptr(ws), nbytes, stream_handle(xh.device)),
+    check(lib().exl3_prefill_matmul_window(ptr(xh), ptr(wt), rows, k, n, n_call, ptr(svh), ptr(bias), ptr(out), ldy,
+                                           DTYPE_CODE[out.dtype], ptr(ws), nbytes, stream_handle(xh.device)),
           "exl3_prefill_matmul")
     return out
 
@@ -450,7 +452,8 @@ def prefill_gemm(xh: torch.Tensor, trellis: torch.Tensor, k: int, n: int, K: int
             w = wt[:cn]
             check(lib().exl3_reconstruct(ptr(trellis), k, n, K, cb, c0 // 16, cn // 16, ptr(w),
                                          stream_handle(xh.device)), "exl3_reconstruct")
-            prefill_matmul(x2, w, svh[c0:c0 + cn], None if bias is None else bias[c0:c0 + cn], y2[:, c0:c0 + cn])
+            prefill_matmul(x2, w, svh[c0:c0 + cn], None if bias is None else bias[c0:c0 + cn], y2[:, c0:c0 + cn],
+                           n_call=n)
         return out
     check(lib().exl3_prefill_gemm(ptr(xh), ptr(trellis), k, n, K, cb, ptr(svh), ptr(bias), ptr(out),
                                   DTYPE_CODE[out_dtype], rows, stream_handle(xh.device)), "exl3_prefill_gemm")
