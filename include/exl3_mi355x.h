@@ -292,7 +292,7 @@ int exl3_attn_decode_rotate(const uint16_t* q, const uint16_t* k, const uint16_t
  *              fine, not shared by calls in flight together; NULL runs exl3_attn_decode_rotate
  *   counters   NULL: a second launch merges; or n_heads x 256 bytes (uint32 every 64 words) zeroed once before the first
  *              use, with the workspace's rules: the last workgroup to arrive merges, in the one launch, and leaves the
- *              counters at zero (the faster form up to a max_len of about 2,048)
+ *              counters at zero (the faster form)
  * Other arguments, cache writes and rounding points as exl3_attn_decode_rotate; the sums over positions are added in
  * another order (fixed by the position and the shape: results are reproducible). */
 int exl3_attn_decode_rotate_ws(const uint16_t* q, const uint16_t* k, const uint16_t* v, uint16_t* k_cache,

@@ -605,27 +605,31 @@ static void launch_attn_split(const dim3& grid, const AttnSplitArgs& a, hipStrea
   attn_split_kernel<GH><<<grid, kAsThreads, (size_t)GH * a.passes * kAsPass * sizeof(float), st>>>(a);
 }
 
-// Head groups of a key/value head and workgroups (S) per head group, from the shape alone. A workgroup's latency grows
-// with its heads (~0.5 us each), so a cache of up to kAsShortLen positions is cut into groups small enough for
-// kAsShortGroups workgroups at full capacity, S leaving kAsShortWorkgroups of them; a longer one is bound by its rows, read
-// once per head group, and takes groups of up to 8 heads and 256 workgroups in all. Measured at 48 / 8 heads, us (position
-// 100 / 700 / capacity - 24): capacity 1024 6.3 / 8.2 / 8.5 (one launch), against 6.5 / 12.3 / 14.1 for one workgroup per
-// head; 2048 6.3 / 8.2 / 11.2 against 6.5 / 12.3 / 21.4; 8192 (two launches) 9.0 / 9.5 / 15.8 against 6.5 / 12.3 / 66.8,
-// where the short plan takes 10.1 / 10.6 / 15.5 and the last-arriver merge 9.9 / 10.5 / 19.4.
-constexpr int kAsShortLen = 2048, kAsShortGroups = 1024, kAsShortWorkgroups = 512, kAsLongWorkgroups = 256;
+// Head groups of a key/value head and workgroups (S) per head group, from the shape alone: one workgroup per CU in all. A
+// workgroup's latency grows with its heads (~0.5 us each) and its passes (~1.4 us each, at most kAsMaxPasses at full
+// capacity: their scores stay in LDS), so the smallest head groups are taken that leave S that many workgroups; more
+// groups than CUs, or more splits, cost more in dispatch and merge than they save. Measured at 48 / 8 heads, us (position 15
+// / 100 / 700 / 2,000 / 4,000 / 8,100), one launch: capacity 1,024 4.5 / 6.4 / 8.2, 4,096 4.9 / 6.9 / 8.2 / 10.8 / 14.4,
+// 8,192 5.2 / 7.5 / 8.3 / 9.9 / 12.7 / 16.5; two launches 2.8 / 1.3 / 1.2 / 1.1 / 1.0 / 0.9 more; one workgroup per head
+// 5.7 / 6.5 / 12.3 / 21.3 / 36.4 / 66. Plans of 512 and 768 workgroups with smaller head groups: up to 0.6 us less at
+// position 100, 3-6 us more at 8,100; groups of up to 8 heads: 2.5 us more at 100.
+constexpr int kAsWorkgroups = 256;
+
+static int attn_least_splits(int max_len) {
+  return (max_len + kAsMaxPasses * kAsPass - 1) / (kAsMaxPasses * kAsPass);
+}
 
 static int attn_head_groups(int n_kv, int grp, int max_len) {
-  const int passes = (max_len + kAsPass - 1) / kAsPass;
-  const int z0 = (grp + kAsMaxHeads - 1) / kAsMaxHeads, least = max_len <= kAsShortLen ? kAsShortGroups : kAsLongWorkgroups;
-  int gh = (grp + z0 - 1) / z0;
-  while (gh > 1 && n_kv * ((grp + gh - 1) / gh) * passes < least) --gh;
+  const int least = attn_least_splits(max_len);
+  int gh = 1;
+  while (gh < grp && gh < kAsMaxHeads && n_kv * ((grp + gh - 1) / gh) * least > kAsWorkgroups) ++gh;
   return (grp + gh - 1) / gh;
 }
 
-// (at least a pass of 64 positions each, at most kAsMaxPasses passes each at full capacity: their scores stay in LDS)
+// (at least a pass of 64 positions each)
 static int attn_splits(int n_kv, int z, int max_len) {
-  const int most = (max_len + kAsPass - 1) / kAsPass, least = (most + kAsMaxPasses - 1) / kAsMaxPasses;
-  const int want = (max_len <= kAsShortLen ? kAsShortWorkgroups : kAsLongWorkgroups) / (n_kv * z);
+  const int most = (max_len + kAsPass - 1) / kAsPass, least = attn_least_splits(max_len);
+  const int want = kAsWorkgroups / (n_kv * z);
   return want > most ? most : want < least ? least : want;
 }
 

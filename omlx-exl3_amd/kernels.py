@@ -461,17 +461,16 @@ def prefill_gemm(xh: torch.Tensor, trellis: torch.Tensor, k: int, n: int, K: int
 
 
 # Decode attention by cache capacity: one workgroup per head up to the first bound; above it the positions are split
-# over workgroups, merged by the last to arrive up to the second bound when the caller holds an attn_workspace, else by
-# a second launch (exl3_attn_decode_rotate_ws; measured sides at csrc/exl3_attn.hip's plan).
+# over workgroups, merged by the last to arrive when the caller holds an attn_workspace, else by a second launch
+# (exl3_attn_decode_rotate_ws; measured sides at csrc/exl3_attn.hip's plan).
 ATTN_UNSPLIT_LEN = 512
-ATTN_WORKSPACE_LEN = 2048
 ATTN_MAX_LEN = 8192
 
 
 def attn_workspace(n_heads: int, n_kv: int, max_len: int, device) -> torch.Tensor | None:
     """A zeroed workspace for attn_decode_rotate calls of this shape that follow each other on one stream (arrival
     counters, left at zero by every call, and the workgroups' sums), or None for a capacity that takes none."""
-    if not ATTN_UNSPLIT_LEN < max_len <= ATTN_WORKSPACE_LEN:
+    if not ATTN_UNSPLIT_LEN < max_len <= ATTN_MAX_LEN:
         return None
     nbytes = lib().exl3_attn_decode_workspace_bytes(n_heads, n_kv, max_len)
     _require(nbytes > 0, "attn_workspace: bad head counts")
@@ -509,7 +508,7 @@ def attn_decode_rotate(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cach
         check(lib().exl3_attn_decode_rotate(*args, stream_handle(q.device)), "exl3_attn_decode_rotate")
         return xh, o
     nbytes = lib().exl3_attn_decode_workspace_bytes(n_heads, n_kv, max_len)
-    if workspace is not None and max_len <= ATTN_WORKSPACE_LEN:
+    if workspace is not None:
         _dev(workspace, "workspace")
         _require(workspace.dtype == torch.uint8 and workspace.numel() == 256 * n_heads + nbytes,
                  "attn_decode_rotate: workspace is attn_workspace of this shape")

@@ -37,11 +37,12 @@ def _rope(x, c, s):
     return torch.cat((lo * c - hi * s, hi * c + lo * s), 1).half()
 
 
-# positions: first, both sides of a 64-position pass and of a workgroup's second pass (48 / 8 heads: 10 workgroups of a
-# head at 1,024 and 2,048, 32 at 8,192), last; head groups of 1, 2, 3, 6 and 8 heads, a group size that does not divide
+# positions: first, both sides of a 64-position pass and of a workgroup's second pass (48 / 8 heads: 5 workgroups of a
+# head at 1,024 and 2,048), last; head groups of 1, 2, 3, 4, 6, 7 and 8 heads, a group size that does not divide
 @pytest.mark.parametrize("n_heads,n_kv,max_len", [(48, 8, 1024), (48, 8, 2048), (48, 8, 8192), (8, 8, 1024),
-                                                 (6, 1, 600), (10, 2, 2048), (64, 4, 4096), (7, 1, 1024)])
-@pytest.mark.parametrize("where", ["0", "63", "64", "640", "639", "-1"])
+                                                 (6, 1, 600), (10, 2, 2048), (64, 4, 4096), (7, 1, 1024),
+                                                 (64, 4, 8192), (96, 16, 8192), (112, 16, 8192), (128, 16, 8192)])
+@pytest.mark.parametrize("where", ["0", "63", "64", "319", "320", "640", "639", "-1"])
 def test_attn_split_vs_torch(pk, n_heads, n_kv, max_len, where):
     pos = int(where) if int(where) >= 0 else max_len - 1
     if pos >= max_len:
