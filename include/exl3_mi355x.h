@@ -175,6 +175,14 @@ int exl3_gemv_fused_mk(int prologue, const uint16_t* x, const uint16_t* residual
                        unsigned flags, const uint16_t* y_residual, double* y_sumsq, void* workspace,
                        size_t workspace_bytes, void* stream);
 
+/* exl3_gemv of rot(x, suh_m) per member, the rotation inside the launch, for fp16 or bf16 x (rows, k) (x_dtype): the values
+ * of exl3_rotate followed by exl3_gemv / exl3_gemv_fused_mk, bit for bit, in one launch. Exact layout, hashing kernel;
+ * member_K as exl3_gemv_fused_mk; suh fp16 (n_members, k); k % 128 == 0; x and suh 16-byte aligned. y must not overlap x,
+ * suh, svh, bias or a trellis. Other arguments as exl3_gemv. */
+int exl3_gemv_rotate(const void* x, int x_dtype, const uint16_t* suh, const uint32_t* const* trellis, int n_members,
+                     const int* member_n, const int* member_K, int k, int cb, const uint16_t* svh, const void* bias,
+                     void* y, int out_dtype, int rows, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Input rotation: xh[m, r, :] = fp16(H128(x[r, :] * suh[m, :]) / sqrt(128)) per 128-block, fp32 inside.
  * Replaces rot (kernels.py:388-406, 451-458). x (rows, k) in x_dtype; suh fp16 (n_members, k);
  * xh fp16 (n_members, rows, k). k % 128 == 0. xh must not overlap x or suh. */

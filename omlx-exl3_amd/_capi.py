@@ -53,6 +53,8 @@ _SIGNATURES = {
                                          _vp, _vp, _vp]),
     "exl3_attn_decode_rotate_ws": (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _c_int,
                                             _vp, _vp, _vp, _vp, _c_size, _vp, _vp]),
+    "exl3_gemv_rotate": (_c_int, [_vp, _c_int, _vp, _vp, _c_int, _vp, _vp, _c_int, _c_int, _vp, _vp, _vp, _c_int, _c_int,
+                                  _vp, _c_size, _vp]),
     "exl3_attn_decode_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int]),
 }
 

@@ -423,6 +423,24 @@ extern "C" int exl3_gemv_fused_mk(int prologue, const uint16_t* x, const uint16_
                         y_sumsq, workspace, workspace_bytes, stream);
 }
 
+extern "C" int exl3_gemv_rotate(const void* x, int x_dtype, const uint16_t* suh, const uint32_t* const* trellis,
+                                int n_members, const int* member_n, const int* member_K, int k, int cb,
+                                const uint16_t* svh, const void* bias, void* y, int out_dtype, int rows, void* workspace,
+                                size_t workspace_bytes, void* stream) {
+  EXL3_REQUIRE(x && suh && member_K, EXL3_ERR_ARG, "exl3_gemv_rotate: NULL pointer argument");
+  EXL3_REQUIRE(x_dtype == kF16 || x_dtype == kBF16, EXL3_ERR_ARG, "exl3_gemv_rotate: x must be fp16 or bf16");
+  EXL3_REQUIRE(n_members >= 1 && n_members <= 3, EXL3_ERR_ARG, "exl3_gemv_rotate: 1..3 members (got %d)", n_members);
+  EXL3_REQUIRE(k > 0 && k % 128 == 0, EXL3_ERR_ARG, "exl3_gemv_rotate: k must be a positive multiple of 128 (got %d)",
+               k);
+  EXL3_REQUIRE(aligned(x, 16) && aligned(suh, 16), EXL3_ERR_ARG,
+               "exl3_gemv_rotate: x and suh must be 16-byte aligned");
+  const GemvPrologueArgs pro{x_dtype == kF16 ? kProRot : kProRotB16,
+                             static_cast<const uint16_t*>(x), nullptr, nullptr, nullptr, nullptr, suh, 0.f, nullptr,
+                             nullptr, nullptr};
+  return gemv_run(nullptr, pro, trellis, n_members, member_n, k, member_K[0], cb, svh, bias, y, out_dtype, rows,
+                  EXL3_GEMV_EXACT, workspace, workspace_bytes, 0, stream, 0, member_K);
+}
+
 extern "C" int exl3_gemv(const uint16_t* xh, const uint32_t* const* trellis, int n_members, const int* member_n,
                          int k, int K, int cb, const uint16_t* svh, const void* bias, void* y, int out_dtype, int rows,
                          unsigned flags, void* workspace, size_t workspace_bytes, void* stream) {

@@ -12,7 +12,8 @@ namespace exl3 {
 // Prologue staging: the split's activations computed in the workgroup from the layer's un-rotated input
 // instead of read from xh. kProNorm: h = fp16(x + residual) and xn = fp16(w * fp16(h * inv_rms)) with the row's
 // sum of squares in fp64 (exact, so independent of the reduction order), as exl3_rmsnorm_rotate computes them;
-// kProSwiglu: silu(gate) * up as exl3_swiglu_rotate computes it; kProRot: x itself. Then e = v * suh_m, the
+// kProSwiglu: silu(gate) * up as exl3_swiglu_rotate computes it; kProRot, kProRotB16: x itself, fp16 or bf16 (fp32 rows are
+// rotated by exl3_rotate: their loads here spilled registers of the K = 6 kernels). Then e = v * suh_m, the
 // 128-point FWHT of each block, * 1/sqrt(128), fp16: the values those kernels (and exl3_rotate) write to xh, so
 // the GEMV's result is bit-identical to rotating first. The workgroup of member 0's first block in each split
 // also writes h and xn for the split's k-range. k is a multiple of 128 (checked on the host).
@@ -77,9 +78,13 @@ __device__ void stage_prologue(const GemvArgs& a, int m, int blk_in_member, int 
     const int kt = c0 >> 4;
     const bool in_split = kt >= kt0 && kt < kt1;
     float v[8];
+    if (a.pro == kProRotB16) {
+      load8<kBF16>(a.px, (size_t)r * k + c0, v);
+    } else {
+      load8<kF16>(a.px, (a.pro == kProSwiglu ? (size_t)r * 2 * k : (size_t)r * k) + c0, v);
+    }
     if (a.pro == kProNorm) {
       float wv[8];
-      load8<kF16>(a.px, (size_t)r * k + c0, v);
       if (a.pres) {
         float rv[8];
         load8<kF16>(a.pres, (size_t)r * k + c0, rv);
@@ -92,11 +97,8 @@ __device__ void stage_prologue(const GemvArgs& a, int m, int blk_in_member, int 
 #pragma unroll
       for (int i = 0; i < 8; ++i) v[i] = round_through<kF16>(wv[i] * round_through<kF16>(v[i] * inv));
       if (write_xn && in_split) store8<kF16>(a.pxn_out, (size_t)r * k + c0, v);
-    } else if (a.pro == kProRot) {
-      load8<kF16>(a.px, (size_t)r * k + c0, v);
-    } else {
+    } else if (a.pro == kProSwiglu) {
       float uv[8];
-      load8<kF16>(a.px, (size_t)r * 2 * k + c0, v);
       load8<kF16>(a.px, (size_t)r * 2 * k + k + c0, uv);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
@@ -144,7 +146,7 @@ __device__ __forceinline__ ProPre prologue_preload(const GemvArgs& a, int m, int
   if (p.valid) {
     const int c0 = (b0 + (tid >> 4)) * 128 + (lane & 15) * 8;
     p.x = *reinterpret_cast<const u32x4*>(a.px + c0);
-    if (a.pro != kProRot) p.w = *reinterpret_cast<const u32x4*>(a.pro == kProNorm ? a.pw + c0 : a.px + k + c0);
+    if (a.pro < kProRot) p.w = *reinterpret_cast<const u32x4*>(a.pro == kProNorm ? a.pw + c0 : a.px + k + c0);
     p.s = *reinterpret_cast<const u32x4*>(a.psuh + (size_t)m * k + c0);
   }
   if (a.pro == kProNorm && tid < k / 128) p.ss = a.pss[tid];
@@ -187,7 +189,13 @@ __device__ void prologue_finish(const GemvArgs& a, const ProPre& p, int kt0, int
   const int c0 = ((kt0 >> 3) + (tid >> 4)) * 128 + (lane & 15) * 8;
   const int kt = c0 >> 4;
   float v[8], w[8], s[8];
-  unpack8(p.x, v);
+  if (a.pro == kProRotB16) {
+    const uint32_t d[4] = {p.x.x, p.x.y, p.x.z, p.x.w};
+#pragma unroll
+    for (int i = 0; i < 8; ++i) v[i] = bf16_to_f32((uint16_t)(d[i / 2] >> (16 * (i % 2))));
+  } else {
+    unpack8(p.x, v);
+  }
   unpack8(p.w, w);
   unpack8(p.s, s);
   if (a.pro == kProNorm) {

@@ -23,7 +23,7 @@ struct GemvArgs {
   int k, KT, rows, n_total, S, kt_per_split;
   // input prologue (kProNone: xh is the rotated input)
   int pro;
-  const uint16_t* px;         // kProNorm, kProRot: x (rows, k); kProSwiglu: gate | up (rows, 2k)
+  const uint16_t* px;         // kProNorm, kProRot, kProRotB16: x (rows, k); kProSwiglu: gate | up (rows, 2k)
   const uint16_t* pres;       // kProNorm: residual (rows, k) or null
   uint16_t* pres_out;         // kProNorm: h = x + residual (rows, k) or null
   uint16_t* pxn_out;          // kProNorm: the norm's output xn (rows, k) or null
@@ -36,7 +36,7 @@ struct GemvArgs {
   double* ess;                // (rows, n_total / 128) or null
 };
 
-enum Prologue : int { kProNone = 0, kProNorm = 1, kProSwiglu = 2, kProRot = 3 };
+enum Prologue : int { kProNone = 0, kProNorm = 1, kProSwiglu = 2, kProRot = 3, kProRotB16 = 4 };
 
 constexpr int kMaxRows = 16;
 constexpr int kCounterStride = 64;   // words between the split-K arrival counters of two blocks (256 bytes)

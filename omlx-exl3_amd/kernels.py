@@ -22,6 +22,12 @@ PROLOGUE_NONE, PROLOGUE_RMSNORM, PROLOGUE_SWIGLU, PROLOGUE_ROTATE = 0, 1, 2, 3  
 MAX_GEMV_ROWS = 8           # rows at or below which EXL3Linear takes the GEMV path (kernels.py:260)
 GEMV_ROWS_LIMIT = 16        # rows one GEMV launch accepts
 GEMV_EXACT, GEMV_FAST, GEMV_TABLE = 0, 1, 2
+# Elements a GEMV launch of several rows rotates inside (every 128-column block rotates its rows again) up to which that
+# beats a rotation launch of its own (~2 us). Measured us, inside / own launch: 6144 -> 5120, 8 rows (2.0 M) 12.5 / 13.9;
+# 5120 -> 2 x 17408, 4 rows (5.6 M) 39.8 / 40.6, 8 rows (11 M) 42.8 / 41.7; 17408 -> 5120, 4 rows (2.8 M) 18.6 / 19.3,
+# 8 rows (5.6 M) 20.8 / 20.4; 5120 -> 151936, 2 / 4 / 8 rows (12 / 24 / 49 M) 134 / 144 / 162 against 130 / 135 / 144. A
+# single row's operands are loaded ahead of the trellis: inside at every shape (5120 -> 151936 129.5 / 133.5).
+ROTATE_IN_LAUNCH_LIMIT = 5_000_000
 
 
 def _require(cond: bool, msg: str) -> None:
@@ -202,6 +208,7 @@ class TrellisGemvPlan:
             nbytes = max(nbytes, self.n // 128 * 256 + (S * rows * self.n * 4 if S > 1 else 0))
         self.workspace = torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=self.device)
         self._ns_c = (ctypes.c_int * 3)(*(list(member_ns) + [0] * (3 - len(member_ns))))
+        self.rotates_inside = rows == 1 or rows * k * (self.n // 128) <= ROTATE_IN_LAUNCH_LIMIT
         self._tr_key = None
         self._tr_c = None
 
@@ -306,6 +313,22 @@ class TrellisGemvPlan:
     def swiglu(self, gu: torch.Tensor, suh: torch.Tensor, trellises: list[torch.Tensor], **kw) -> torch.Tensor:
         """fused(PROLOGUE_SWIGLU, ...): the GEMV of rot(silu(gate) * up, suh) with gu = [gate | up]."""
         return self.fused(PROLOGUE_SWIGLU, gu, trellises, suh=suh, **kw)
+
+    def rotate_bf16(self, x: torch.Tensor, suh: torch.Tensor, trellises: list[torch.Tensor], *,
+                    bias: torch.Tensor | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
+        """rotate for bf16 x (exl3_gemv_rotate): the values of rot followed by __call__, in one launch."""
+        _dev(x, "x")
+        _dev(suh, "suh")
+        _require(x.dtype == torch.bfloat16 and x.numel() == self.rows * self.k, f"x must be bf16 ({self.rows}, {self.k})")
+        _require(suh.dtype == torch.float16 and suh.numel() == self.nsub * self.k, "suh: fp16 (n_members, k)")
+        _require(self.flags == GEMV_EXACT and not self.kt_per_split, "rotate_bf16: the default plan only")
+        out = self._bind(trellises, bias, out, x.device)
+        self._check_y(out, [x, suh, bias, *trellises])
+        check(lib().exl3_gemv_rotate(ptr(x), DTYPE_CODE[x.dtype], ptr(suh), self._tr_c, self.nsub, self._ns_c, self._Ks_c,
+                                     self.k, self.cb, ptr(self.svh), ptr(bias), ptr(out), DTYPE_CODE[self.out_dtype],
+                                     self.rows, ptr(self.workspace), self.workspace.numel(), stream_handle(x.device)),
+              "exl3_gemv_rotate")
+        return out
 
     def rotate(self, x: torch.Tensor, suh: torch.Tensor, trellises: list[torch.Tensor], **kw) -> torch.Tensor:
         """fused(PROLOGUE_ROTATE, ...): the GEMV of rot(x, suh_m) per member, the rotation inside the launch

@@ -301,6 +301,9 @@ class EXL3Linear(nn.Module):
                                                    [self._tr], bias=bias, y_residual=y_res, y_sumsq=y_ss)
                 if armed:
                     self._armed_out = y
+            elif xh is None and dtype == torch.bfloat16 and self._armed is None and self._plan(rows, dtype).rotates_inside:
+                y = self._plan(rows, dtype).rotate_bf16(x.reshape(rows, self.in_features).contiguous(), self._suh2d,
+                                                        [self._tr], bias=bias)
             else:
                 if xh is None:
                     xh = rot(x.reshape(rows, self.in_features).contiguous(), self._suh2d)
@@ -373,11 +376,13 @@ class EXL3SiblingGroup:
 
     def gemv(self, x: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
         """All members' outputs, concatenated: (rows, sum(ns)) in out_dtype (rows <= MAX_GEMV_ROWS). The input
-        rotations run inside the GEMV launch for fp16 input, unless a rotated input was primed."""
+        rotations run inside the GEMV launch for fp16 and bf16 input, unless a rotated input was primed."""
         rows = x.numel() // self.k
         xh = self._primed.take(x)
         if xh is None and x.dtype == torch.float16:
             return self._plan(rows, out_dtype).rotate(x.reshape(rows, self.k).contiguous(), self.suh, self.trs)
+        if xh is None and x.dtype == torch.bfloat16 and self._plan(rows, out_dtype).rotates_inside:
+            return self._plan(rows, out_dtype).rotate_bf16(x.reshape(rows, self.k).contiguous(), self.suh, self.trs)
         if xh is None:
             xh = rot(x.reshape(rows, self.k).contiguous(), self.suh)
         return self._plan(rows, out_dtype)(xh.contiguous(), self.trs)
