@@ -293,7 +293,8 @@ class EXL3Linear(nn.Module):
         bias = self._bias_for(dtype)
         if rows <= MAX_GEMV_ROWS:
             xh = self._primed.take(x)
-            if xh is None and dtype == torch.float16:
+            inside = xh is None and self._plan(rows, dtype).rotates_inside
+            if inside and dtype == torch.float16:
                 # the input rotation inside the GEMV launch (exl3_gemv_fused, ROTATE prologue)
                 armed = self._armed is not None
                 y_res, y_ss = self._take_arm(rows, dtype)
@@ -301,7 +302,7 @@ class EXL3Linear(nn.Module):
                                                    [self._tr], bias=bias, y_residual=y_res, y_sumsq=y_ss)
                 if armed:
                     self._armed_out = y
-            elif xh is None and dtype == torch.bfloat16 and self._armed is None and self._plan(rows, dtype).rotates_inside:
+            elif inside and dtype == torch.bfloat16 and self._armed is None:
                 y = self._plan(rows, dtype).rotate_bf16(x.reshape(rows, self.in_features).contiguous(), self._suh2d,
                                                         [self._tr], bias=bias)
             else:
@@ -376,16 +377,16 @@ class EXL3SiblingGroup:
 
     def gemv(self, x: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
         """All members' outputs, concatenated: (rows, sum(ns)) in out_dtype (rows <= MAX_GEMV_ROWS). The input
-        rotations run inside the GEMV launch for fp16 and bf16 input, unless a rotated input was primed."""
+        rotations run inside the GEMV launch for fp16 and bf16 input up to a measured amount, unless a rotated input was primed."""
         rows = x.numel() // self.k
         xh = self._primed.take(x)
-        if xh is None and x.dtype == torch.float16:
-            return self._plan(rows, out_dtype).rotate(x.reshape(rows, self.k).contiguous(), self.suh, self.trs)
-        if xh is None and x.dtype == torch.bfloat16 and self._plan(rows, out_dtype).rotates_inside:
-            return self._plan(rows, out_dtype).rotate_bf16(x.reshape(rows, self.k).contiguous(), self.suh, self.trs)
+        plan = self._plan(rows, out_dtype)
+        if xh is None and plan.rotates_inside and x.dtype in (torch.float16, torch.bfloat16):
+            rotate = plan.rotate if x.dtype == torch.float16 else plan.rotate_bf16
+            return rotate(x.reshape(rows, self.k).contiguous(), self.suh, self.trs)
         if xh is None:
             xh = rot(x.reshape(rows, self.k).contiguous(), self.suh)
-        return self._plan(rows, out_dtype)(xh.contiguous(), self.trs)
+        return plan(xh.contiguous(), self.trs)
 
     def gemv_rmsnorm(self, x: torch.Tensor, residual: torch.Tensor | None, weight: torch.Tensor, eps: float,
                      out_dtype: torch.dtype, residual_out: torch.Tensor | None = None,
