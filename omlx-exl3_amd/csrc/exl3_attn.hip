@@ -358,11 +358,13 @@ __global__ __launch_bounds__(kAsThreads) void attn_split_kernel(AttnSplitArgs a)
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     m[r] = fmaxf(fmaxf(sm[0][4 * q + r], sm[1][4 * q + r]), fmaxf(sm[2][4 * q + r], sm[3][4 * q + r]));
+    // (a range of scores that are all -inf adds nothing: exp(-inf - 0), not exp(-inf + inf))
+    const float mr = m[r] == -INFINITY ? 0.f : m[r];
     float l = 0.f;
     if (4 * q + r < GH) {
       for (int j = 0; j < passes; ++j) {
         float& x = sp[(4 * q + r) * pitch + j * kAsPass + wave * 16 + c];
-        const float e = expf(x - m[r]);
+        const float e = expf(x - mr);
         x = e;
         l += e;
       }

@@ -86,3 +86,21 @@ def test_attn_split_workspace_of_another_shape_is_refused(pk):
     ws = pk.kernels.attn_workspace(8, 2, 1024, "cuda")
     with pytest.raises(ValueError):
         pk.kernels.attn_decode_rotate(q, k, v, kc, vc, p, cos, sin, suh, workspace=ws)
+
+
+@pytest.mark.parametrize("n_heads,n_kv", [(48, 8), (8, 8), (7, 1)])
+def test_attn_split_workgroup_of_minus_infinity_scores(pk, n_heads, n_kv):
+    """A 64-position pass whose scores are all -inf has probability zero, as with one workgroup per head."""
+    pos, max_len = 300, 1024
+    q, k, v, kc, vc, p, cos, sin, suh = _inputs(n_heads, n_kv, pos, max_len)
+    cos[pos], sin[pos] = 1.0, 0.0
+    q.view(-1, 128)[:, 0] = 1.0
+    kc[:, 64:128, 0] = -math.inf
+    keep = [i for i in range(pos) if not 64 <= i < 128]
+    K = torch.cat((kc[:, keep], k.view(-1, 1, 128)), 1).double()
+    V = torch.cat((vc[:, keep], v.view(-1, 1, 128)), 1).double()
+    sc = torch.matmul(q.double().view(n_kv, -1, 128), K.transpose(1, 2).contiguous()) / math.sqrt(128)
+    ref = torch.matmul(torch.softmax(sc, -1), V).reshape(-1)
+    for ws in (None, pk.kernels.attn_workspace(n_heads, n_kv, max_len, "cuda")):
+        _, o = pk.kernels.attn_decode_rotate(q, k, v, kc.clone(), vc.clone(), p, cos, sin, suh, want_o=True, workspace=ws)
+        assert ((o.view(-1).double() - ref).abs().max() / ref.abs().max()).item() < 1e-3
