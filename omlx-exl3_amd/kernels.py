@@ -27,7 +27,9 @@ GEMV_EXACT, GEMV_FAST, GEMV_TABLE = 0, 1, 2
 # 5120 -> 2 x 17408, 4 rows (5.6 M) 39.8 / 40.6, 8 rows (11 M) 42.8 / 41.7; 17408 -> 5120, 4 rows (2.8 M) 18.6 / 19.3,
 # 8 rows (5.6 M) 20.8 / 20.4; 5120 -> 151936, 2 / 4 / 8 rows (12 / 24 / 49 M) 134 / 144 / 162 against 130 / 135 / 144. A
 # single row's operands are loaded ahead of the trellis: inside at every shape (5120 -> 151936 129.5 / 133.5).
-ROTATE_IN_LAUNCH_LIMIT = 5_000_000
+# The limit lies above the level pair of 17408 -> 5120: a call that launches twice also takes the host longer than a
+# 20 us launch takes the GPU (3-bit, 8 rows, a call among others: 21.1 us inside, 25.1 with a launch of its own).
+ROTATE_IN_LAUNCH_LIMIT = 8_000_000
 
 
 def _require(cond: bool, msg: str) -> None:

@@ -53,15 +53,15 @@ def test_bf16_linear_is_one_launch(pk, monkeypatch):
 
 @pytest.mark.parametrize("rows,inside", [(1, True), (4, True), (8, False)])
 def test_linear_on_both_sides_of_the_rotation_rule(pk, rows, inside):
-    """17408 -> 5120: one launch and two launches give rot followed by the GEMV bit for bit, armed or not."""
+    """17408 -> 7680: one launch and two launches give rot followed by the GEMV bit for bit, armed or not."""
     syn = importlib.import_module(pk.__name__ + ".synthetic")
     g = torch.Generator(device="cuda").manual_seed(rows)
-    lin = syn.random_exl3_linear(17408, 5120, 2, 0, g, "cuda")
+    lin = syn.random_exl3_linear(17408, 7680, 2, 0, g, "cuda")
     for dt in (torch.float16, torch.bfloat16):
         x = torch.randn(rows, 17408, device="cuda", generator=g).to(dt)
         assert lin._plan(rows, dt).rotates_inside == inside
         assert torch.equal(lin(x), lin.gemv_rotated(pk.kernels.rot(x, lin.rot_suh), dt))
-    x, res = x.half(), torch.randn(rows, 5120, device="cuda", generator=g).half()
+    x, res = x.half(), torch.randn(rows, 7680, device="cuda", generator=g).half()
     y = lin(x)
     lin.arm_residual(res)
     assert torch.equal(lin(x), (y.float() + res.float()).half()) and lin.take_armed_output() is not None
