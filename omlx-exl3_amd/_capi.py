@@ -90,7 +90,9 @@ def check(rc: int, what: str) -> None:
 
 def stream_handle(device: torch.device | None = None) -> int:
     """The current torch stream of `device` as a raw hipStream_t."""
-    return torch.cuda.current_stream(device).cuda_stream
+    if device is None or device.index is None:
+        return torch.cuda.current_stream(device).cuda_stream
+    return torch._C._cuda_getCurrentRawStream(device.index)      # (without a Stream object for every call)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

@@ -38,8 +38,10 @@ def _require(cond: bool, msg: str) -> None:
 
 
 def _dev(t: torch.Tensor, name: str) -> None:
-    _require(isinstance(t, torch.Tensor) and t.is_cuda, f"{name} must be a tensor on the HIP device")
-    _require(t.is_contiguous(), f"{name} must be contiguous")
+    if not (isinstance(t, torch.Tensor) and t.is_cuda):
+        raise ValueError(f"{name} must be a tensor on the HIP device")
+    if not t.is_contiguous():
+        raise ValueError(f"{name} must be contiguous")
 
 
 def _overlap(a: torch.Tensor | None, b: torch.Tensor | None) -> bool:
@@ -61,14 +63,16 @@ def _check_vec(t: torch.Tensor | None, n: int, dtype: torch.dtype, name: str) ->
     if t is None:
         return
     _dev(t, name)
-    _require(t.dtype == dtype and t.numel() == n, f"{name} must be {dtype} with {n} elements, got {t.dtype} {t.numel()}")
+    if not (t.dtype == dtype and t.numel() == n):
+        raise ValueError(f"{name} must be {dtype} with {n} elements, got {t.dtype} {t.numel()}")
 
 
 def trellis_words(trellis: torch.Tensor, k: int, n: int, K: int) -> torch.Tensor:
     """Check a trellis tensor (int16 [k/16, n/16, 16K], or any contiguous tensor of those bytes)."""
     _dev(trellis, "trellis")
     nbytes = trellis.numel() * trellis.element_size()
-    _require(nbytes == k * n * K // 8, f"trellis holds {nbytes} bytes, expected k*n*K/8 = {k * n * K // 8}")
+    if nbytes != k * n * K // 8:
+        raise ValueError(f"trellis holds {nbytes} bytes, expected k*n*K/8 = {k * n * K // 8}")
     return trellis
 
 
@@ -319,23 +323,50 @@ class TrellisGemvPlan:
     def rotate_bf16(self, x: torch.Tensor, suh: torch.Tensor, trellises: list[torch.Tensor], *,
                     bias: torch.Tensor | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
         """rotate for bf16 x (exl3_gemv_rotate): the values of rot followed by __call__, in one launch."""
-        _dev(x, "x")
-        _dev(suh, "suh")
-        _require(x.dtype == torch.bfloat16 and x.numel() == self.rows * self.k, f"x must be bf16 ({self.rows}, {self.k})")
-        _require(suh.dtype == torch.float16 and suh.numel() == self.nsub * self.k, "suh: fp16 (n_members, k)")
         _require(self.flags == GEMV_EXACT and not self.kt_per_split, "rotate_bf16: the default plan only")
-        out = self._bind(trellises, bias, out, x.device)
-        self._check_y(out, [x, suh, bias, *trellises])
+        out = self._rotate_args(x, torch.bfloat16, suh, trellises, bias, out)
         check(lib().exl3_gemv_rotate(ptr(x), DTYPE_CODE[x.dtype], ptr(suh), self._tr_c, self.nsub, self._ns_c, self._Ks_c,
                                      self.k, self.cb, ptr(self.svh), ptr(bias), ptr(out), DTYPE_CODE[self.out_dtype],
                                      self.rows, ptr(self.workspace), self.workspace.numel(), stream_handle(x.device)),
               "exl3_gemv_rotate")
         return out
 
-    def rotate(self, x: torch.Tensor, suh: torch.Tensor, trellises: list[torch.Tensor], **kw) -> torch.Tensor:
+    def rotate(self, x: torch.Tensor, suh: torch.Tensor, trellises: list[torch.Tensor], *,
+               bias: torch.Tensor | None = None, out: torch.Tensor | None = None,
+               y_residual: torch.Tensor | None = None, y_sumsq: torch.Tensor | None = None, **kw) -> torch.Tensor:
         """fused(PROLOGUE_ROTATE, ...): the GEMV of rot(x, suh_m) per member, the rotation inside the launch
         (the same values as rot followed by __call__)."""
-        return self.fused(PROLOGUE_ROTATE, x, trellises, suh=suh, **kw)
+        if kw or y_residual is not None or y_sumsq is not None:
+            return self.fused(PROLOGUE_ROTATE, x, trellises, suh=suh, bias=bias, out=out, y_residual=y_residual,
+                              y_sumsq=y_sumsq, **kw)
+        out = self._rotate_args(x, torch.float16, suh, trellises, bias, out)
+        if self.mixed:
+            rc = lib().exl3_gemv_fused_mk(PROLOGUE_ROTATE, ptr(x), None, None, None, None, 0.0, None, ptr(suh), self._tr_c,
+                                          self.nsub, self._ns_c, self._Ks_c, self.k, self.cb, ptr(self.svh), ptr(bias),
+                                          ptr(out), DTYPE_CODE[self.out_dtype], self.rows, self.flags, None, None,
+                                          ptr(self.workspace), self.workspace.numel(), stream_handle(x.device))
+            check(rc, "exl3_gemv_fused_mk")
+            return out
+        check(lib().exl3_gemv_fused(PROLOGUE_ROTATE, ptr(x), None, None, None, None, 0.0, None, ptr(suh), self._tr_c,
+                                    self.nsub, self._ns_c, self.k, self.K, self.cb, ptr(self.svh), ptr(bias), ptr(out),
+                                    DTYPE_CODE[self.out_dtype], self.rows, self.flags, None, None, ptr(self.workspace),
+                                    self.workspace.numel(), stream_handle(x.device)), "exl3_gemv_fused")
+        return out
+
+    def _rotate_args(self, x: torch.Tensor, dtype: torch.dtype, suh: torch.Tensor, trellises: list[torch.Tensor],
+                     bias: torch.Tensor | None, out: torch.Tensor | None) -> torch.Tensor:
+        """The checks of a call without an epilogue, and its output. A small layer spends longer in its host lines than
+        on the GPU, so only what this call can get wrong is looked at (an output made here shares no memory with
+        anything): a one-row call of 4096^2 at 4 bits took 18.3 us through fused, and takes 10.0."""
+        if not (x.is_cuda and x.is_contiguous() and x.dtype == dtype and x.numel() == self.rows * self.k):
+            raise ValueError(f"x must be a contiguous {dtype} tensor ({self.rows}, {self.k}) on the HIP device")
+        if not (suh.is_cuda and suh.is_contiguous() and suh.dtype == torch.float16 and suh.numel() == self.nsub * self.k):
+            raise ValueError("suh must be a contiguous fp16 tensor (n_members, k) on the HIP device")
+        given = out is not None
+        out = self._bind(trellises, bias, out, x.device)
+        if given:
+            self._check_y(out, [x, suh, bias, *trellises])
+        return out
 
 
 def prefill_matmul(xh: torch.Tensor, wt: torch.Tensor, svh: torch.Tensor, bias: torch.Tensor | None,
@@ -378,6 +409,11 @@ def prefill_rows(xh: torch.Tensor, trellis: torch.Tensor, k: int, n: int, K: int
     trellis_words(trellis, k, n, K)
     _check_vec(svh, n, torch.float16, "svh")
     _check_vec(bias, n, out.dtype, "bias")
+    return _prefill_rows(xh, trellis, k, n, K, cb, svh, bias, out, rows, splits)
+
+
+def _prefill_rows(xh, trellis, k, n, K, cb, svh, bias, out, rows, splits):
+    """prefill_rows' launch, its arguments checked by the caller."""
     nbytes = lib().exl3_prefill_rows_workspace_bytes(rows, k, n, K, splits)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=xh.device) if nbytes else None
     check(lib().exl3_prefill_rows(ptr(xh), ptr(trellis), k, n, K, cb, ptr(svh), ptr(bias), ptr(out),
@@ -455,7 +491,9 @@ def prefill_gemm(xh: torch.Tensor, trellis: torch.Tensor, k: int, n: int, K: int
     _require(path in PREFILL_PATHS, f"prefill_gemm: unknown path {path!r}")
     _require(out_dtype in DTYPE_CODE, "prefill_gemm: out_dtype fp16, bf16 or fp32")
     trellis_words(trellis, k, n, K)
-    svh = svh.to(torch.float16).reshape(-1).contiguous()
+    if svh.dtype != torch.float16 or svh.dim() != 1:
+        svh = svh.to(torch.float16).reshape(-1)
+    svh = svh.contiguous()
     _check_vec(svh, n, torch.float16, "svh")
     _check_vec(bias, n, out_dtype, "bias")
     if out is None:
@@ -463,13 +501,14 @@ def prefill_gemm(xh: torch.Tensor, trellis: torch.Tensor, k: int, n: int, K: int
     else:
         _check_out(out, (rows, n), out_dtype)
         _require(not _overlap(out, xh), "prefill_gemm: out must not overlap xh")
-    rows_form = path == "auto" and takes_rows_form(rows, k, n, K)
+    if path == "auto" and takes_rows_form(rows, k, n, K):
+        if 2 * _CHUNK_ALIGN * k > min(chunk_bytes, _GEMM_OPERAND_LIMIT - 1):
+            prefill_chunks(n, k, chunk_bytes)           # refuses the caller's bound, as for the reconstruction
+        return _prefill_rows(xh, trellis, k, n, K, cb, svh, bias, out, rows, 0)
     if path == "auto":
         path = "matmul" if k % 64 == 0 else "fused"
     if path == "matmul":
-        chunks = prefill_chunks(n, k, chunk_bytes)     # (also the rows form's check of the caller's bound)
-        if rows_form:
-            return prefill_rows(xh, trellis, k, n, K, cb, svh, bias, out)
+        chunks = prefill_chunks(n, k, chunk_bytes)
         x2 = xh.reshape(rows, k).contiguous()
         y2 = out.view(rows, n)
         wt = torch.empty((chunks[0][1], k), dtype=torch.float16, device=xh.device)

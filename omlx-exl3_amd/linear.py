@@ -293,22 +293,22 @@ class EXL3Linear(nn.Module):
         bias = self._bias_for(dtype)
         if rows <= MAX_GEMV_ROWS:
             xh = self._primed.take(x)
-            inside = xh is None and self._plan(rows, dtype).rotates_inside
-            if inside and dtype == torch.float16:
-                # the input rotation inside the GEMV launch (exl3_gemv_fused, ROTATE prologue)
+            plan = self._plan(rows, dtype)
+            if xh is None and plan.rotates_inside and dtype == torch.float16:
+                # the input rotation inside the GEMV launch (ROTATE prologue)
                 armed = self._armed is not None
                 y_res, y_ss = self._take_arm(rows, dtype)
-                y = self._plan(rows, dtype).rotate(x.reshape(rows, self.in_features).contiguous(), self._suh2d,
-                                                   [self._tr], bias=bias, y_residual=y_res, y_sumsq=y_ss)
+                y = plan.rotate(x.contiguous(), self._suh2d, [self._tr], bias=bias, y_residual=y_res, y_sumsq=y_ss)
                 if armed:
                     self._armed_out = y
-            elif inside and dtype == torch.bfloat16 and self._armed is None:
-                y = self._plan(rows, dtype).rotate_bf16(x.reshape(rows, self.in_features).contiguous(), self._suh2d,
-                                                        [self._tr], bias=bias)
+            elif xh is None and plan.rotates_inside and dtype == torch.bfloat16 and self._armed is None:
+                y = plan.rotate_bf16(x.contiguous(), self._suh2d, [self._tr], bias=bias)
             else:
                 if xh is None:
                     xh = rot(x.reshape(rows, self.in_features).contiguous(), self._suh2d)
                 y = self.gemv_rotated(xh, dtype, bias)
+            if len(in_shape) == 2:
+                return y
         else:
             xh = rot(x.reshape(rows, self.in_features).contiguous(), self._suh2d).reshape(rows, self.in_features)
             y = self._prefill(xh, dtype, bias)
@@ -383,7 +383,7 @@ class EXL3SiblingGroup:
         plan = self._plan(rows, out_dtype)
         if xh is None and plan.rotates_inside and x.dtype in (torch.float16, torch.bfloat16):
             rotate = plan.rotate if x.dtype == torch.float16 else plan.rotate_bf16
-            return rotate(x.reshape(rows, self.k).contiguous(), self.suh, self.trs)
+            return rotate(x.contiguous(), self.suh, self.trs)
         if xh is None:
             xh = rot(x.reshape(rows, self.k).contiguous(), self.suh)
         return plan(xh.contiguous(), self.trs)
