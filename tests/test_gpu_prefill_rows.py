@@ -3,6 +3,8 @@
 Bars: an fp32 result differs from the fp64 oracle by fp32 accumulation alone (products of fp16 values are exact in
 fp32), at most k * 2^-24 of the largest result (k <= 1088: 6.5e-5, bar 1e-4); fp16 and bf16 results add their
 rounding, twice with a bias (2e-3, 1e-2: the bars of the other prefill forms)."""
+import importlib
+
 import numpy as np
 import pytest
 
@@ -90,3 +92,24 @@ def test_prefill_auto_route(pk, rows, k, n):
     want = _run(pk, tr, svh, xh, k, n, K, 0, torch.float32) if rows_form else \
         pk.kernels.prefill_gemm(xh, tr, k, n, K, 0, svh, out_dtype=torch.float32, path="matmul")
     assert torch.equal(y, want) and O.max_abs_rel(y.cpu().numpy(), ref) < BAR[torch.float32]
+
+
+# three members of different widths and bits; a strided input; both prefill forms (k = 1024: rows form up to 640 rows)
+@pytest.mark.parametrize("rows", [9, 33, 700])
+@pytest.mark.parametrize("dt", ["float16", "bfloat16", "float32"])
+def test_group_prefill_equals_its_members(pk, rows, dt):
+    syn = importlib.import_module(pk.__name__ + ".synthetic")
+    lin_mod = importlib.import_module(pk.__name__ + ".linear")
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    lins = [syn.random_exl3_linear(1024, n, K, 0, g, "cuda") for n, K in ((1280, 5), (256, 6), (128, 8))]
+    x = torch.randn(2, rows, 1024, device="cuda", generator=g).to(getattr(torch, dt)).transpose(0, 1)
+    want = [lin(x) for lin in lins]
+    group = lin_mod.EXL3SiblingGroup(lins)
+    for got, w in zip(group(x), want):
+        assert got.shape == w.shape and got.dtype == w.dtype and torch.equal(got, w)
+    calls = []
+    hook = lins[1].register_forward_hook(lambda *a: calls.append(1))
+    assert all(torch.equal(a, b) for a, b in zip(group(x), want)) and calls
+    hook.remove()
+    with pytest.raises(ValueError):
+        group(x.reshape(-1, 512))
