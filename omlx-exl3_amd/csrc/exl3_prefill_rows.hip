@@ -2,6 +2,8 @@
 // Entry point and launch plan of the few-row prefill; the kernels and what bounds them: exl3_prefill_rows_body.h.
 #include "exl3_prefill_rows.h"
 
+#include <algorithm>
+
 #include "exl3_capi_common.h"
 #include "exl3_device.h"
 #include "exl3_prefill_reduce.h"
@@ -41,7 +43,8 @@ static RowsPlan rows_plan(int rows, int k, int n, int splits) {
     const int rt = rows_rt((rows + z - 1) / z);
     if (z > z0 && rt < 4) break;   // (smaller tiles decode more often than they spread the work)
     if ((rows + 16 * rt - 1) / (16 * rt) != z) continue;   // the same row blocks as a smaller z
-    const int s_lo = splits > 0 ? splits : 1, s_hi = splits > 0 ? splits : kMaxSplits;
+    // (a step per split at most; steps + S - 1 below stays in range for any `splits`)
+    const int s_lo = splits > 0 ? std::min(splits, steps) : 1, s_hi = splits > 0 ? s_lo : kMaxSplits;
     for (int S = s_lo; S <= s_hi; ++S) {
       const int per = (steps + S - 1) / S;
       if (splits <= 0 && S > 1 && per < 3) break;

@@ -277,3 +277,16 @@ def test_prefill_rows_argument_errors(capi):
     assert lib.exl3_prefill_rows_workspace_bytes(9, 512, 256, 6, 1) == 0
     assert lib.exl3_prefill_rows_workspace_bytes(9, 512, 256, 6, 100) == 8 * 9 * 256 * 4   # one step per split at most
     assert lib.exl3_prefill_rows_workspace_bytes(9, 500, 256, 6, 2) == 0                   # invalid shape
+
+
+def test_prefill_rows_split_count_past_int_range(capi):
+    """Any split count, the largest int among them, means one step per split at most (it once overflowed to a division
+    by zero)."""
+    lib = capi.lib()
+    p = ctypes.c_void_p(0x10000)
+    for k, steps in ((64, 1), (512, 8), (17408, 272)):
+        want = steps * 9 * 256 * 4 if steps > 1 else 0
+        for splits in (steps, steps + 1, 1 << 20, (1 << 31) - steps, (1 << 31) - 1):
+            assert lib.exl3_prefill_rows_workspace_bytes(9, k, 256, 6, splits) == want, (k, splits)
+        if want:
+            assert lib.exl3_prefill_rows(p, p, k, 256, 6, 0, p, None, p, 0, 9, (1 << 31) - 1, None, 0, None) == -2
