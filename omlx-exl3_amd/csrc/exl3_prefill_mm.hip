@@ -379,14 +379,12 @@ __global__ __launch_bounds__(kMmThreads) __attribute__((amdgpu_waves_per_eu(2)))
 // tile, the pair of least estimated time. A round of w workgroups (256 at most, one per CU) takes, per 64-k step of a
 // split, a[ti] + b[ti] w / 256 us (the more CUs work, the lower the clock), and f[ti] besides; S > 1 adds the reduction
 // launch: 1.2 + 0.31 S us and S + 1 passes over an fp32 rows x n array at 3.16 TB/s (2.3 TB/s beyond 48 MB), and a
-// workspace of S x rows x n fp32, held to kMmWorkspaceLimit. At least 4 steps per split, S <= 16. The constants were
+// workspace of S x rows x n fp32, held to kPrefillWorkspaceLimit. At least 4 steps per split, S <= 16. The constants were
 // fitted to 111 shapes (k 1,024-17,408, n 512-17,408, 200-4,608 rows) x 3 heights x up to 8 splits, over which the pick
 // is on average within 2% of the fastest measured pair (4% for the rule before, which picked the height first and split
 // launches of at most 128 tiles). The sides, us before / now: 17408 -> 5120 at 777 / 1,024 / 1,300 rows 218 / 233 / 234
 // against 153 / 166 / 215; 5120 -> 1024 at 777 / 1,024 rows 28.5 / 33.5 against 22.9 / 24.4; 8192 -> 1024 at 3,000 rows 70
 // against 59; the largest loss, 5120 -> 1024 at 1,300 rows, 28.2 against 29.6.
-constexpr size_t kMmWorkspaceLimit = (size_t)128 << 20;
-
 struct MmPlan {
   int ti, tiles_m, splits, steps_per_split;
 };
@@ -404,7 +402,7 @@ static MmPlan mm_plan(int rows, int k, int n) {
     const long tiles = (long)tiles_m * tiles_n;
     for (int S = 1; S <= 16; ++S) {
       const int sps = (nsteps + S - 1) / S;
-      if (S > 1 && (sps < 4 || tiles * S > 1024 || S * out_bytes > (double)kMmWorkspaceLimit)) break;
+      if (S > 1 && (sps < 4 || tiles * S > 1024 || S * out_bytes > (double)kPrefillWorkspaceLimit)) break;
       if ((nsteps + sps - 1) / sps != S) continue;   // an S that leaves an empty split: the plan of a smaller one
       const long groups = tiles * S, rest = groups % 256;
       auto round_us = [&](long w) { return sps * (a[ti - 2] + b[ti - 2] * (double)w / 256.0) + f[ti - 2]; };

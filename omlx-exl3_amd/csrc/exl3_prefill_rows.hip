@@ -14,7 +14,8 @@ namespace exl3 {
 // estimated from what was measured at 7 shapes (k 1,024-17,408, n 1,024-17,408) x 15 row counts x up to 13 splits: a
 // 64-k step of a workgroup costs 0.195 + 0.0355 RT us when others share its CU, at least 0.21 + 0.055 RT alone (latency),
 // kRowsResident workgroups fit a CU, ~6.3 us are fixed, and the splits' sums are written and read once at ~6.4 TB/s
-// plus a second launch. Over those shapes the pick is within 4% of the best measured plan except at a few small ones.
+// plus a second launch. Automatic plans split while the sums stay within kPrefillWorkspaceLimit (a wide head has column
+// blocks enough: 92 rows of 17408 -> 151936 took 160 MiB of sums, 246 rows 428 MiB). Over those shapes the pick is within 4% of the best measured plan except at a few small ones.
 struct RowsPlan {
   int rt, row_blocks, splits, kt_per_split;
 };
@@ -47,7 +48,9 @@ static RowsPlan rows_plan(int rows, int k, int n, int splits) {
     const int s_lo = splits > 0 ? std::min(splits, steps) : 1, s_hi = splits > 0 ? s_lo : kMaxSplits;
     for (int S = s_lo; S <= s_hi; ++S) {
       const int per = (steps + S - 1) / S;
-      if (splits <= 0 && S > 1 && per < 3) break;
+      if (splits <= 0 && S > 1 &&
+          (per < 3 || (size_t)S * (size_t)rows * (size_t)n * sizeof(float) > kPrefillWorkspaceLimit))
+        break;
       const int real = (steps + per - 1) / per;   // no empty split
       const double us = rows_cost(rt, (long)(n / 128) * z, per, real, (double)rows * n * 4.0);
       if (best_us < 0 || us < best_us) {

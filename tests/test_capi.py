@@ -290,3 +290,17 @@ def test_prefill_rows_split_count_past_int_range(capi):
             assert lib.exl3_prefill_rows_workspace_bytes(9, k, 256, 6, splits) == want, (k, splits)
         if want:
             assert lib.exl3_prefill_rows(p, p, k, 256, 6, 0, p, None, p, 0, 9, (1 << 31) - 1, None, 0, None) == -2
+
+
+def test_prefill_rows_workspace_is_bounded(capi):
+    """Automatic plans hold the splits' sums to 128 MiB, however wide the output; a caller's own split count stands."""
+    lib = capi.lib()
+    sizes = []
+    for k in (1024, 5120, 17408):
+        for n in (5120, 17408, 65536, 151936):
+            for rows in (9, 33, 92, 211, 246, 512, 640, 1024):
+                b = lib.exl3_prefill_rows_workspace_bytes(rows, k, n, 1, 0)
+                assert b % (rows * n * 4) == 0
+                sizes.append(b)
+    assert 0 < max(sizes) <= 128 << 20
+    assert lib.exl3_prefill_rows_workspace_bytes(246, 17408, 151936, 1, 3) == 3 * 246 * 151936 * 4
