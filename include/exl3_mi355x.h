@@ -189,6 +189,10 @@ int exl3_gemv_rotate(const void* x, int x_dtype, const uint16_t* suh, const uint
 int exl3_rotate(const void* x, int x_dtype, const uint16_t* suh, int n_members, int rows, int k, uint16_t* xh,
                 void* stream);
 
+/* exl3_rotate with each member's scales in a buffer of its own: suh[m] fp16 (k), 16-byte aligned, n_members 1..3. */
+int exl3_rotate_members(const void* x, int x_dtype, const uint16_t* const* suh, int n_members, int rows, int k,
+                        uint16_t* xh, void* stream);
+
 /* Fused residual add + RMSNorm + input rotations. Replaces norm_rot (kernels.py:408-425, 461-473) and
  * the residual add the reference leaves to the model graph.
  *   h  = T(x + residual)   when residual != NULL (written to residual_out if non-NULL), else h = x

@@ -35,6 +35,7 @@ _SIGNATURES = {
                                     _c_int, _c_int, _vp, _vp, _vp, _c_int, _c_int, _c_uint, _vp, _vp, _vp, _c_size,
                                     _vp]),
     "exl3_rotate": (_c_int, [_vp, _c_int, _vp, _c_int, _c_int, _c_int, _vp, _vp]),
+    "exl3_rotate_members": (_c_int, [_vp, _c_int, _vp, _c_int, _c_int, _c_int, _vp, _vp]),
     "exl3_rmsnorm_rotate": (_c_int, [_vp, _vp, _vp, _vp, _c_int, _c_float, _vp, _c_int, _c_int, _c_int, _vp, _vp,
                                      _vp]),
     "exl3_swiglu_rotate": (_c_int, [_vp, _vp, _c_int, _c_int, _vp, _vp]),

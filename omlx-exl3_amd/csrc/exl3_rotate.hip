@@ -13,13 +13,21 @@
 
 namespace exl3 {
 
+// The members' input scales: rows of one (n_members, k) array, or (more == true) up to three vectors of their own.
+struct RotScales {
+  const uint16_t *suh, *suh1, *suh2;
+  bool more;
+  __device__ __forceinline__ const uint16_t* of(int m, int k) const {
+    return !more ? suh + (size_t)m * k : m == 0 ? suh : m == 1 ? suh1 : suh2;
+  }
+};
+
 // rotate the 8 values of this lane (element offset c0 within the row) for every member and store to xh
-__device__ __forceinline__ void rotate_members(const float (&xv)[8], const uint16_t* __restrict__ suh, int nm,
-                                               int rows, int r, int k, size_t c0, uint16_t* __restrict__ xh,
-                                               int lane, bool valid) {
+__device__ __forceinline__ void rotate_members(const float (&xv)[8], const RotScales& suh, int nm, int rows, int r,
+                                               int k, size_t c0, uint16_t* __restrict__ xh, int lane, bool valid) {
   for (int m = 0; m < nm; ++m) {
     float e[8], s[8];
-    if (valid) load8<kF16>(suh, (size_t)m * k + c0, s);
+    if (valid) load8<kF16>(suh.of(m, k), c0, s);
     else {
 #pragma unroll
       for (int i = 0; i < 8; ++i) s[i] = 0.f;
@@ -35,8 +43,8 @@ __device__ __forceinline__ void rotate_members(const float (&xv)[8], const uint1
 
 // grid (ceil(k / 2048), rows), 256 threads: each thread owns 8 consecutive elements
 template <int DT>
-__global__ __launch_bounds__(256) void rot_kernel(const void* __restrict__ x, const uint16_t* __restrict__ suh,
-                                                  int nm, int rows, int k, uint16_t* __restrict__ xh) {
+__global__ __launch_bounds__(256) void rot_kernel(const void* __restrict__ x, RotScales suh, int nm, int rows, int k,
+                                                  uint16_t* __restrict__ xh) {
   const int lane = threadIdx.x & 63;
   const int r = blockIdx.y;
   const size_t c0 = ((size_t)blockIdx.x * 256 + threadIdx.x) * 8;
@@ -114,7 +122,7 @@ __global__ __launch_bounds__(256) void norm_rot_kernel(const void* __restrict__ 
 #pragma unroll
       for (int i = 0; i < 8; ++i) xv[i] = 0.f;
     }
-    rotate_members(xv, suh, nm, rows, r, k, c0, xh, lane, valid);
+    rotate_members(xv, RotScales{suh, nullptr, nullptr, false}, nm, rows, r, k, c0, xh, lane, valid);
   }
 }
 
@@ -152,28 +160,44 @@ __global__ __launch_bounds__(256) void swiglu_rot_kernel(const uint16_t* __restr
 
 using namespace exl3;
 
-extern "C" int exl3_rotate(const void* x, int x_dtype, const uint16_t* suh, int n_members, int rows, int k,
-                           uint16_t* xh, void* stream) {
-  EXL3_REQUIRE(x && suh && xh, EXL3_ERR_ARG, "exl3_rotate: NULL pointer argument");
-  EXL3_REQUIRE(k > 0 && k % 128 == 0, EXL3_ERR_ARG, "exl3_rotate: k must be a positive multiple of 128 (got %d)", k);
-  EXL3_REQUIRE(rows >= 1 && rows <= 65535, EXL3_ERR_ARG, "exl3_rotate: rows must be 1..65535 (got %d)", rows);
-  EXL3_REQUIRE(n_members >= 1, EXL3_ERR_ARG, "exl3_rotate: n_members must be >= 1 (got %d)", n_members);
-  EXL3_REQUIRE(x_dtype >= 0 && x_dtype <= 2, EXL3_ERR_ARG, "exl3_rotate: bad x_dtype %d", x_dtype);
-  EXL3_REQUIRE(aligned(x, 16) && aligned(suh, 16) && aligned(xh, 16), EXL3_ERR_ARG,
-               "exl3_rotate: x, suh and xh must be 16-byte aligned");
-  {
-    const size_t xb = (size_t)rows * k * (x_dtype == kF32 ? 4 : 2);
-    const size_t hb = (size_t)n_members * rows * k * 2;
-    EXL3_REQUIRE(!overlaps(xh, hb, x, xb) && !overlaps(xh, hb, suh, (size_t)n_members * k * 2), EXL3_ERR_ARG,
-                 "exl3_rotate: xh must not overlap x or suh");
+static int rotate_run(const char* what, const void* x, int x_dtype, const RotScales& suh, int n_members, int rows, int k,
+                      uint16_t* xh, void* stream) {
+  EXL3_REQUIRE(k > 0 && k % 128 == 0, EXL3_ERR_ARG, "%s: k must be a positive multiple of 128 (got %d)", what, k);
+  EXL3_REQUIRE(rows >= 1 && rows <= 65535, EXL3_ERR_ARG, "%s: rows must be 1..65535 (got %d)", what, rows);
+  EXL3_REQUIRE(x_dtype >= 0 && x_dtype <= 2, EXL3_ERR_ARG, "%s: bad x_dtype %d", what, x_dtype);
+  EXL3_REQUIRE(aligned(x, 16) && aligned(xh, 16), EXL3_ERR_ARG, "%s: x, suh and xh must be 16-byte aligned", what);
+  const size_t xb = (size_t)rows * k * (x_dtype == kF32 ? 4 : 2), hb = (size_t)n_members * rows * k * 2;
+  EXL3_REQUIRE(!overlaps(xh, hb, x, xb), EXL3_ERR_ARG, "%s: xh must not overlap x or suh", what);
+  for (int m = 0; m < (suh.more ? n_members : 1); ++m) {
+    const uint16_t* s = m == 0 ? suh.suh : m == 1 ? suh.suh1 : suh.suh2;
+    EXL3_REQUIRE(aligned(s, 16), EXL3_ERR_ARG, "%s: x, suh and xh must be 16-byte aligned", what);
+    EXL3_REQUIRE(!overlaps(xh, hb, s, (size_t)(suh.more ? 1 : n_members) * k * 2), EXL3_ERR_ARG,
+                 "%s: xh must not overlap x or suh", what);
   }
   hipStream_t st = static_cast<hipStream_t>(stream);
   const dim3 grid((unsigned)((k + 2047) / 2048), (unsigned)rows);
   if (x_dtype == kF16) rot_kernel<kF16><<<grid, 256, 0, st>>>(x, suh, n_members, rows, k, xh);
   else if (x_dtype == kBF16) rot_kernel<kBF16><<<grid, 256, 0, st>>>(x, suh, n_members, rows, k, xh);
   else rot_kernel<kF32><<<grid, 256, 0, st>>>(x, suh, n_members, rows, k, xh);
-  EXL3_LAUNCH_CHECK("exl3_rotate");
+  EXL3_LAUNCH_CHECK(what);
   return EXL3_OK;
+}
+
+extern "C" int exl3_rotate(const void* x, int x_dtype, const uint16_t* suh, int n_members, int rows, int k,
+                           uint16_t* xh, void* stream) {
+  EXL3_REQUIRE(x && suh && xh, EXL3_ERR_ARG, "exl3_rotate: NULL pointer argument");
+  EXL3_REQUIRE(n_members >= 1, EXL3_ERR_ARG, "exl3_rotate: n_members must be >= 1 (got %d)", n_members);
+  return rotate_run("exl3_rotate", x, x_dtype, RotScales{suh, nullptr, nullptr, false}, n_members, rows, k, xh, stream);
+}
+
+extern "C" int exl3_rotate_members(const void* x, int x_dtype, const uint16_t* const* suh, int n_members, int rows, int k,
+                                   uint16_t* xh, void* stream) {
+  EXL3_REQUIRE(n_members >= 1 && n_members <= 3, EXL3_ERR_ARG, "exl3_rotate_members: 1..3 members (got %d)", n_members);
+  EXL3_REQUIRE(x && suh && xh, EXL3_ERR_ARG, "exl3_rotate_members: NULL pointer argument");
+  for (int m = 0; m < n_members; ++m)
+    EXL3_REQUIRE(suh[m], EXL3_ERR_ARG, "exl3_rotate_members: NULL suh of member %d", m);
+  const RotScales s{suh[0], suh[n_members > 1 ? 1 : 0], suh[n_members > 2 ? 2 : 0], true};
+  return rotate_run("exl3_rotate_members", x, x_dtype, s, n_members, rows, k, xh, stream);
 }
 
 extern "C" int exl3_rmsnorm_rotate(const void* x, const void* residual, void* residual_out, const void* w, int dtype,

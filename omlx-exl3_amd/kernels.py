@@ -117,6 +117,20 @@ def rot(x: torch.Tensor, suh: torch.Tensor, out: torch.Tensor | None = None) -> 
     return out
 
 
+def rot_members(x: torch.Tensor, suhs: list[torch.Tensor]) -> torch.Tensor:
+    """rot for one to three members whose scales (k,) fp16 lie in tensors of their own (exl3_rotate_members):
+    (n_members, rows, k) fp16."""
+    _dev(x, "x")
+    rows, k = x.shape
+    _require(x.dtype in DTYPE_CODE and 1 <= len(suhs) <= 3, "rot_members: x must be fp16/bf16/fp32, 1..3 members")
+    for s in suhs:
+        _check_vec(s, k, torch.float16, "suh")
+    out = torch.empty((len(suhs), rows, k), dtype=torch.float16, device=x.device)
+    check(lib().exl3_rotate_members(ptr(x), DTYPE_CODE[x.dtype], (ctypes.c_void_p * 3)(*map(ptr, suhs)), len(suhs), rows, k,
+                                    ptr(out), stream_handle(x.device)), "exl3_rotate_members")
+    return out
+
+
 def norm_rot(x: torch.Tensor, w: torch.Tensor, eps: float, suh: torch.Tensor | None,
              residual: torch.Tensor | None = None, residual_out: torch.Tensor | None = None):
     """RMSNorm(x [+ residual]) * w in x.dtype (MLX's rounding) and its rotations xh (NM, rows, k) fp16
@@ -586,6 +600,6 @@ def attn_decode_rotate(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cach
     return xh, o
 
 
-__all__ = ["MAX_GEMV_ROWS", "GEMV_ROWS_LIMIT", "TrellisGemvPlan", "decode_wt", "rot", "norm_rot", "swiglu_rot",
+__all__ = ["MAX_GEMV_ROWS", "GEMV_ROWS_LIMIT", "TrellisGemvPlan", "decode_wt", "rot", "rot_members", "norm_rot", "swiglu_rot",
            "prefill_gemm", "prefill_chunks", "prefill_matmul", "prefill_rows", "takes_rows_form", "prefill_out_rotate", "PREFILL_CHUNK_BYTES", "codebook",
            "attn_decode_rotate", "attn_workspace", "Exl3Error"]

@@ -33,8 +33,9 @@ import math
 import torch
 import torch.nn.functional as F
 from torch import nn
+from torch.nn.modules.module import _has_any_global_hook
 
-from .kernels import MAX_GEMV_ROWS, PROLOGUE_NONE, TrellisGemvPlan, prefill_gemm, rot
+from .kernels import MAX_GEMV_ROWS, PROLOGUE_NONE, TrellisGemvPlan, prefill_gemm, rot, rot_members
 
 _HAD_SCALE = 1.0 / math.sqrt(128.0)
 EXL3_PARTS = ("trellis", "suh", "svh", "su", "sv", "mul1", "mcg", "bias")
@@ -279,6 +280,13 @@ class EXL3Linear(nn.Module):
         return prefill_gemm(xh, self._tr, self.in_features, self.out_features, self._K, self._cb, self._svh,
                             bias=bias, out_dtype=out_dtype)
 
+    def _call_is_forward(self) -> bool:
+        """Whether calling this module runs EXL3Linear.forward and nothing else (no hook, subclass, replaced or compiled
+        forward, no output computed ahead), so that a caller may do forward's steps itself."""
+        return (type(self) is EXL3Linear and "forward" not in self.__dict__ and self._served.key is None
+                and self._compiled_call_impl is None and not _has_any_global_hook()
+                and not (self._forward_hooks or self._forward_pre_hooks or self._backward_hooks or self._backward_pre_hooks))
+
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self._group is not None:
             return self._group.member_output(x, self._idx)
@@ -420,15 +428,16 @@ class EXL3SiblingGroup:
         y = self._served.take(x)
         if y is not None:
             return tuple(o.reshape(in_shape[:-1] + (n,)) for o, n in zip(torch.split(y, self.ns, dim=-1), self.ns))
-        if rows > MAX_GEMV_ROWS and x.shape[-1] == self.k and not any(
-                m._served.key is not None or m._forward_hooks or m._forward_pre_hooks for m in self.members):
+        if rows > MAX_GEMV_ROWS and x.shape[-1] == self.k and all(m._call_is_forward() for m in self.members):
             # prefill: the input rotated for every member in one launch, which reads it once (5120 columns, two members,
             # us: 33 / 211 / 4,608 rows 2.7 / 4.2 / 35 against 4.5 / 6.1 / 47 in two; a bf16 MLP of 211 rows 218.9 -> 215.9),
-            # then each member's product
-            xh = rot(x.reshape(rows, self.k).contiguous(), self.suh)
+            # then each member's product. The members' own scales: theirs may have been loaded or moved since grouping.
+            for m in self.members:
+                m._prepare()
+            xh = rot_members(x.reshape(rows, self.k).contiguous(), [m._suh for m in self.members])
             out = tuple(m._prefill(xh[i], dtype, None).reshape(in_shape[:-1] + (n,))
                         for i, (m, n) in enumerate(zip(self.members, self.ns)))
-        elif rows > MAX_GEMV_ROWS:   # (an output computed ahead for a member, its hooks, its error: its own path)
+        elif rows > MAX_GEMV_ROWS:   # (an output computed ahead for a member, its hooks or own forward, its error)
             outs = []
             for m in self.members:
                 m._group = None

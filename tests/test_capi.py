@@ -304,3 +304,20 @@ def test_prefill_rows_workspace_is_bounded(capi):
                 sizes.append(b)
     assert 0 < max(sizes) <= 128 << 20
     assert lib.exl3_prefill_rows_workspace_bytes(246, 17408, 151936, 1, 3) == 3 * 246 * 151936 * 4
+
+
+def test_rotate_members_argument_errors(capi):
+    lib = capi.lib()
+    p = ctypes.c_void_p(0x100000)
+
+    def rm(x=p, suh=(0x10000, 0x20000, 0x30000), nm=3, rows=9, k=256, xh=ctypes.c_void_p(0x200000)):
+        return lib.exl3_rotate_members(x, 0, suh and (ctypes.c_void_p * 3)(*suh), nm, rows, k, xh, None)
+
+    assert rm(nm=0) == -1 and rm(nm=4) == -1 and "1..3 members" in _err(capi)
+    assert rm(x=None) == -1 and rm(suh=None) == -1 and rm(xh=None) == -1 and "NULL" in _err(capi)
+    assert rm(suh=(0x10000, 0, 0x30000)) == -1 and "member 1" in _err(capi)
+    assert rm(k=192) == -1 and "128" in _err(capi)
+    assert rm(rows=0) == -1 and rm(rows=65536) == -1 and "rows" in _err(capi)
+    assert rm(suh=(0x10000, 0x20000, 0x30008)) == -1 and "aligned" in _err(capi)
+    assert rm(suh=(0x10000, 0x20000, 0x200100)) == -1 and "overlap" in _err(capi)
+    assert rm(xh=ctypes.c_void_p(0x100100)) == -1 and "overlap" in _err(capi)

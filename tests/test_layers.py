@@ -398,3 +398,64 @@ def test_fusion_binds_transformers_llama_layers():
     # the layer's keyword arguments reach the attention module unchanged
     kw = step._mixer_kwargs(torch.zeros(1, 1, 256), (), {"attention_mask": None, "position_ids": 3})
     assert kw == {"attention_mask": None, "position_ids": 3}
+
+
+def _fill(lin, seed):
+    g = torch.Generator().manual_seed(seed)
+    return {k: (torch.randint(-9, 9, v.shape, generator=g).to(v.dtype) if v.dtype == torch.int16
+                else torch.randn(v.shape, generator=g).to(v.dtype)) for k, v in lin.state_dict().items()}
+
+
+@pytest.mark.parametrize("change", ["none", "load_state_dict", "data", "apply", "subclass", "forward", "hook", "pre_hook",
+                                    "global_hook", "compiled", "served"])
+def test_group_prefill_follows_its_members(monkeypatch, change):
+    """A grouped prefill gives what calling each member gives, whatever became of a member after grouping: scales loaded
+    in place, a moved module, a subclass, a replaced forward, hooks. (Stand-ins for the kernels: any function of the
+    rotated input, the trellis and the scales tells members and their tensors apart.)"""
+    k, ns, rows = 256, (128, 256), 12
+    monkeypatch.setattr(linear, "rot", lambda x, suh: (x.float() * suh.float()[:, None]).half())
+    monkeypatch.setattr(linear, "rot_members", lambda x, s: torch.stack([(x.float() * v.float()).half() for v in s]),
+                        raising=False)
+    monkeypatch.setattr(linear, "prefill_gemm", lambda xh, tr, k, n, K, cb, svh, bias=None, out_dtype=None:
+                        (xh.float().sum(-1, keepdim=True) * svh.float() + tr.float().sum()).to(out_dtype))
+
+    class Own(linear.EXL3Linear):
+        def forward(self, x):
+            return super().forward(x) * 2
+    cls = Own if change == "subclass" else linear.EXL3Linear
+    lins = [cls(k, n, _parts(k, n, 4)) for n in ns]
+    for i, lin in enumerate(lins):
+        lin.load_state_dict(_fill(lin, i))
+    group = linear.EXL3SiblingGroup(lins)
+    x, seen, handle = torch.randn(rows, k, generator=torch.Generator().manual_seed(7)).half(), [], None
+    group(x)
+    m = lins[1]
+    if change == "load_state_dict":
+        m.load_state_dict(_fill(m, 11))
+    elif change == "data":
+        m.suh.data.copy_(_fill(m, 12)["suh"])
+    elif change == "apply":
+        m._apply(lambda t: t.clone() * 2)
+    elif change == "forward":
+        m.forward = lambda x, f=m.forward: f(x) * 2
+    elif change == "hook":
+        handle = m.register_forward_hook(lambda mod, a, y: seen.append(1) or y * 3)
+    elif change == "pre_hook":
+        handle = m.register_forward_pre_hook(lambda mod, a: seen.append(1))
+    elif change == "global_hook":
+        handle = nn.modules.module.register_module_forward_hook(lambda mod, a, y: seen.append(1) or y * 3)
+    elif change == "compiled":
+        m._compiled_call_impl = lambda x: seen.append(1) or m.forward(x)
+    elif change == "served":
+        m.serve(x, torch.full((rows, ns[1]), 5.0).half())
+    try:
+        got = group(x)
+        assert change not in ("hook", "pre_hook", "global_hook", "compiled") or seen
+        group.ungroup()
+        if change == "served":
+            m.serve(x, torch.full((rows, ns[1]), 5.0).half())
+        for a, lin in zip(got, lins):
+            assert torch.equal(a, lin(x))
+    finally:
+        if handle is not None:
+            handle.remove()
