@@ -15,6 +15,8 @@
 // k and v rows itself (identical bytes) before reading the caches, so no workgroup depends on another's
 // writes. The position is read from device memory, so a captured graph advances it without host work; a
 // position outside [0, max_len) writes nothing and yields zeros.
+#include <algorithm>
+
 #include "exl3_capi_common.h"
 #include "exl3_device.h"
 
@@ -201,8 +203,11 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(
 // positions 64 (j S + s) ..) of one key/value head for a group of its query heads, so a long context spreads over the
 // chip, and the workgroups' results are merged: by the last one to arrive when arrival counters are given, else by a
 // second launch. The launch is sized by max_len (known to the host), the position is read on the device: workgroups past
-// it end at once. Bound by latency: the chain position -> rows and rotary operands -> scores -> softmax -> P V -> merge
-// (4.4 us for one pass of one head group in one launch), plus ~1.4 us per further pass.
+// it end at once, and while there are few positions (AttnSplitArgs::direct) the first workgroups of a head group take a
+// head each with all its passes, write the outputs themselves, and nothing is merged. Bound by latency: the chain
+// position -> rows and rotary operands -> scores -> softmax -> P V -> merge (4.8 us for one pass of one head), plus
+// 0.85 us per further pass of one head, ~1.1 of three; issue-bound by then: rows loaded two passes ahead instead of one
+// were level or slower (8,192 positions: 16.0 -> 16.5 us).
 //   scores: v_mfma_f32_16x16x32_f16, A = the query heads (rows past them are never used), B = 16 cached rows as their
 //     lanes load them from memory (lane 16q + c: row c, dimensions 32 s + 8 q ..), so keys pass through no LDS
 //   softmax of the workgroup's positions in fp32, probabilities in LDS, P V on the VALU in fp32 (lane 16 q + c:
@@ -230,6 +235,7 @@ struct AttnSplitArgs {
   const int64_t* pos;
   const float *rcos, *rsin;
   int grp, max_len, splits, passes;   // passes: the most 64-position passes of a workgroup
+  int direct;                         // positions below it are held by one workgroup per head
   float scale;
   float* part_o;    // (n_heads, splits, 128): the range's sum of exp(s - m) v
   float2* part_ml;  // (n_heads, splits): its m and sum of exp(s - m)
@@ -239,8 +245,16 @@ struct AttnSplitArgs {
 };
 constexpr int kAsCounterStride = 64;
 
+// What a workgroup of the split form does: nh query heads from h0 on of key/value head kh, the passes at base, base +
+// stride, ... . n: workgroups that hold positions of these heads (1: this one writes their outputs). part: its place among
+// them; group: the arrival counter; adds_row: it writes the new key/value rows if it holds their position.
+struct AttnWork {
+  int kh, h0, nh, base, stride, n, part, group;
+  bool adds_row;
+};
+
 template <int GH>
-__global__ __launch_bounds__(kAsThreads) void attn_split_kernel(AttnSplitArgs a) {
+__device__ __forceinline__ void attn_split_body(const AttnSplitArgs& a, const AttnWork& wk, int pos) {
   extern __shared__ float sp[];   // [GH][64 x passes]: scores, then exp(s - m), of this workgroup's positions
   __shared__ __align__(16) uint16_t sq[16 * kAsPitch];
   __shared__ __align__(16) uint16_t sk[kAttnHD], sv[kAttnHD];
@@ -248,25 +262,10 @@ __global__ __launch_bounds__(kAsThreads) void attn_split_kernel(AttnSplitArgs a)
   __shared__ float sm[kAsWaves][16], sl[kAsWaves][16];
   __shared__ float sw[GH][128], sf[GH][kAttnHD];   // the merge's weights; the heads' outputs
   __shared__ uint32_t arrived_last;
-  const int64_t pos64 = *a.pos;
-  const int base = blockIdx.x * kAsPass, stride = a.splits * kAsPass;
-  const int hz = blockIdx.z * GH;
-  if (a.counters && (pos64 < 0 || pos64 >= (int64_t)a.max_len)) {   // an invalid position yields zeros
-    if (blockIdx.x == 0)
-      for (int idx = threadIdx.x; idx < min(GH, a.grp - hz) * kAttnHD; idx += kAsThreads) {
-        const size_t at = (size_t)(blockIdx.y * a.grp + hz) * kAttnHD + idx;
-        if (a.o) a.o[at] = 0;
-        if (a.xh) a.xh[at] = 0;
-      }
-    return;
-  }
-  // (uniform; without counters an invalid position leaves every workgroup idle and the second launch writes the zeros)
-  if (pos64 < base || pos64 >= (int64_t)a.max_len || hz >= a.grp) return;
-  const int pos = (int)pos64, L = pos + 1;
-  const int passes = (pos - base) / stride + 1, pitch = a.passes * kAsPass;
-  const int kh = blockIdx.y, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int base = wk.base, stride = wk.stride, kh = wk.kh, h0 = wk.h0, nh = wk.nh, n = wk.n;
+  const int L = pos + 1, passes = (pos - base) / stride + 1, pitch = a.passes * kAsPass;
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int q = lane >> 4, c = lane & 15;
-  const int nh = min(GH, a.grp - hz), h0 = kh * a.grp + hz;
   const size_t kv0 = (size_t)kh * a.max_len * kAttnHD;
   const int last = max(pos - 1, 0);   // (rows from pos on are replaced or masked below)
 
@@ -316,7 +315,7 @@ __global__ __launch_bounds__(kAsThreads) void attn_split_kernel(AttnSplitArgs a)
   }
   if (has_new && tid < kAttnHD) sv[tid] = a.v[(size_t)kh * kAttnHD + tid];
   __syncthreads();
-  if (has_new && blockIdx.z == 0 && tid < 32) {   // the new rows, once per key/value head
+  if (has_new && wk.adds_row && tid < 32) {   // the new rows, once per key/value head
     const int e = tid & 15;
     uint16_t* dst = (tid < 16 ? a.kc : a.vc) + kv0 + (size_t)pos * kAttnHD;
     reinterpret_cast<u32x4*>(dst)[e] = reinterpret_cast<const u32x4*>(tid < 16 ? sk : sv)[e];
@@ -425,8 +424,7 @@ __global__ __launch_bounds__(kAsThreads) void attn_split_kernel(AttnSplitArgs a)
     *reinterpret_cast<float2*>(&so[wave][h][8 * c + 4 * (q >> 1) + 2 * (q & 1)]) = float2{r2[0], r2[1]};
   }
   __syncthreads();
-  const int n = min(pos / kAsPass + 1, a.splits);   // workgroups with positions
-  if (n == 1 && a.counters) {   // this one holds them all
+  if (n == 1) {   // this one holds them all
     for (int idx = tid; idx < nh * kAttnHD; idx += kAsThreads) {
       const int h = idx >> 7, d = idx & 127;
       const float l = ((sl[0][h] + sl[1][h]) + sl[2][h]) + sl[3][h];
@@ -439,12 +437,12 @@ __global__ __launch_bounds__(kAsThreads) void attn_split_kernel(AttnSplitArgs a)
   // device-scope stores: with counters, the last workgroup to arrive reads them in this launch
   for (int idx = tid; idx < nh * kAttnHD; idx += kAsThreads) {
     const int h = idx >> 7, d = idx & 127;
-    __hip_atomic_store(a.part_o + ((size_t)(h0 + h) * a.splits + blockIdx.x) * kAttnHD + d,
+    __hip_atomic_store(a.part_o + ((size_t)(h0 + h) * a.splits + wk.part) * kAttnHD + d,
                        ((so[0][h][d] + so[1][h][d]) + so[2][h][d]) + so[3][h][d], __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
   }
   if (tid < nh) {
-    float* ml = reinterpret_cast<float*>(a.part_ml + (size_t)(h0 + tid) * a.splits + blockIdx.x);
+    float* ml = reinterpret_cast<float*>(a.part_ml + (size_t)(h0 + tid) * a.splits + wk.part);
     __hip_atomic_store(ml, fmaxf(fmaxf(sm[0][tid], sm[1][tid]), fmaxf(sm[2][tid], sm[3][tid])), __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
     __hip_atomic_store(ml + 1, ((sl[0][tid] + sl[1][tid]) + sl[2][tid]) + sl[3][tid], __ATOMIC_RELAXED,
@@ -454,7 +452,7 @@ __global__ __launch_bounds__(kAsThreads) void attn_split_kernel(AttnSplitArgs a)
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this thread's stores are acknowledged
   __syncthreads();
   if (tid == 0) {
-    uint32_t* ctr = a.counters + (size_t)(kh * gridDim.z + blockIdx.z) * kAsCounterStride;
+    uint32_t* ctr = a.counters + (size_t)wk.group * kAsCounterStride;
     const uint32_t prev = __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     arrived_last = prev == (uint32_t)(n - 1);
     if (arrived_last) __hip_atomic_store(ctr, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // zero again at rest
@@ -542,29 +540,63 @@ __global__ __launch_bounds__(kAsThreads) void attn_split_kernel(AttnSplitArgs a)
   for (int h = wave; h < nh; h += kAsWaves) write_head(sf[h], h0 + h, lane, a.suh, a.o, a.xh);
 }
 
+template <int GH>
+__global__ __launch_bounds__(kAsThreads) void attn_split_kernel(AttnSplitArgs a) {
+  const int64_t pos64 = *a.pos;
+  // the arguments used past the first branch, loaded with the position's address instead of where they are used
+  asm volatile("" ::"s"(a.q), "s"(a.kc), "s"(a.rcos), "s"(a.direct), "s"(a.scale), "s"(a.part_o), "s"(a.counters), "s"(a.o));
+  const int x = blockIdx.x, kh = blockIdx.y, hz = blockIdx.z * GH;
+  const int h0 = kh * a.grp + hz, nh = min(GH, a.grp - hz);
+  if (pos64 < 0 || pos64 >= (int64_t)a.max_len) {   // an invalid position yields zeros
+    if (x == 0)
+      for (int idx = threadIdx.x; idx < nh * kAttnHD; idx += kAsThreads) {
+        const size_t at = (size_t)h0 * kAttnHD + idx;
+        if (a.o) a.o[at] = 0;
+        if (a.xh) a.xh[at] = 0;
+      }
+    return;
+  }
+  const int pos = (int)pos64, group = kh * gridDim.z + blockIdx.z;
+  AttnWork wk{kh, h0, nh, x * kAsPass, a.splits * kAsPass, min(pos / kAsPass + 1, a.splits), x, group, blockIdx.z == 0};
+  if (pos < a.direct) {   // few positions: a workgroup per head holds them all
+    if (x >= nh) return;
+    wk = AttnWork{kh, h0 + x, 1, 0, kAsPass, 1, 0, group, blockIdx.z == 0 && x == 0};
+    if constexpr (GH > 1) {
+      attn_split_body<1>(a, wk, pos);
+      return;
+    }
+  }
+  if (wk.base > pos || nh <= 0) return;
+  attn_split_body<GH>(a, wk, pos);
+}
+
 // Adds a head's workgroups (at most 128) and writes o and its rotation, as the one-launch form does. Thread (g, e) adds
 // workgroups g, g + 16, ... of dimensions 4 e .. 4 e + 3, all loads of a thread in flight together (two threads per
-// dimension with eight loads each, in batches: 2.6 us more at 64 workgroups). Every slot is loaded before the position is
-// known; the slots past the workgroups in use hold anything and are not added.
+// dimension with eight loads each, in batches: 2.6 us more at 64 workgroups; loads only of the slots there are, a branch
+// each: 0.25 us more, the first is waited for alone). Every slot is loaded before the position is known; the slots past
+// the workgroups in use hold anything and are not added.
 constexpr int kAmThreads = 512, kAmGroups = kAmThreads / 32, kAmLoads = 8;
 
 __global__ __launch_bounds__(kAmThreads) void attn_merge_kernel(const float* __restrict__ part_o,
                                                                 const float2* __restrict__ part_ml,
                                                                 const int64_t* __restrict__ pos_p, int max_len,
-                                                                int splits, const uint16_t* __restrict__ suh,
+                                                                int direct, int splits, const uint16_t* __restrict__ suh,
                                                                 uint16_t* __restrict__ o_out, uint16_t* __restrict__ xh) {
   __shared__ float sw[128], red[4], sfin[kAttnHD];
   __shared__ f32x4 so[kAmGroups][32];
   const int h = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int e = tid & 31, g = tid >> 5;
+  const int64_t pos64 = *pos_p;
   const f32x4* po = reinterpret_cast<const f32x4*>(part_o + (size_t)h * splits * kAttnHD) + e;
   f32x4 t[kAmLoads];
 #pragma unroll
   for (int u = 0; u < kAmLoads; ++u)
-    if (u * kAmGroups < splits) t[u] = po[(size_t)min(g + u * kAmGroups, splits - 1) * 32];
+    t[u] = po[(size_t)min(g + u * kAmGroups, splits - 1) * 32];
   const float2 ml = part_ml[(size_t)h * splits + min(tid, splits - 1)];
-  const int64_t pos64 = *pos_p;
-  const int n = pos64 >= 0 && pos64 < (int64_t)max_len ? min((int)(pos64 / kAsPass) + 1, splits) : 0;
+  asm volatile("" ::"v"(ml.x), "v"(ml.y));   // (every load ahead of the branch)
+  // (the first launch wrote the outputs: of few positions, and the zeros of an invalid one)
+  if (pos64 < (int64_t)direct || pos64 < kAsPass || pos64 >= (int64_t)max_len || splits == 1) return;
+  const int n = min((int)(pos64 / kAsPass) + 1, splits);
   float mx = 0.f, w = 0.f;
   if (wave < 2) {   // the weights exp(m - max m) of up to 128 workgroups, by two wavefronts
     mx = tid < n ? ml.x : -INFINITY;
@@ -596,7 +628,7 @@ __global__ __launch_bounds__(kAmThreads) void attn_merge_kernel(const float* __r
     float o = 0.f;
 #pragma unroll
     for (int u = 0; u < kAmGroups; ++u) o += reinterpret_cast<const float*>(so[u])[tid];
-    sfin[tid] = n > 0 ? round_f16(o / (red[2] + red[3])) : 0.f;
+    sfin[tid] = round_f16(o / (red[2] + red[3]));
   }
   __syncthreads();
   if (wave == 0) write_head(sfin, h, lane, suh, o_out, xh);
@@ -608,13 +640,20 @@ static void launch_attn_split(const dim3& grid, const AttnSplitArgs& a, hipStrea
 }
 
 // Head groups of a key/value head and workgroups (S) per head group, from the shape alone: one workgroup per CU in all. A
-// workgroup's latency grows with its heads (~0.5 us each) and its passes (~1.4 us each, at most kAsMaxPasses at full
-// capacity: their scores stay in LDS), so the smallest head groups are taken that leave S that many workgroups; more
-// groups than CUs, or more splits, cost more in dispatch and merge than they save. Measured at 48 / 8 heads, us (position 15
-// / 100 / 700 / 2,000 / 4,000 / 8,100), one launch: capacity 1,024 4.5 / 6.4 / 8.2, 4,096 4.9 / 6.9 / 8.2 / 10.8 / 14.4,
-// 8,192 5.2 / 7.5 / 8.3 / 9.9 / 12.7 / 16.5; two launches 2.8 / 1.3 / 1.2 / 1.1 / 1.0 / 0.9 more; one workgroup per head
-// 5.7 / 6.5 / 12.3 / 21.3 / 36.4 / 66. Plans of 512 and 768 workgroups with smaller head groups: up to 0.6 us less at
-// position 100, 3-6 us more at 8,100; groups of up to 8 heads: 2.5 us more at 100.
+// workgroup's latency grows with its heads (~0.5 us each) and its passes (at most kAsMaxPasses at full capacity: their
+// scores stay in LDS), so the smallest head groups are taken that leave S that many workgroups; more groups than CUs, or
+// more splits, cost more in dispatch and merge than they save. Measured at 48 / 8 heads, us, graph replays of one call
+// (rows in the caches from the replay before; in a decode step, among the layers' weights, 9.6 at position 700 of 1,024),
+// position 15 / 100 / 200 / 300 / 700 / 2,000 / 4,000 / 8,100:
+//   one launch, capacity 1,024    4.8 / 5.9 / 7.0 / 7.3 / 8.4
+//               capacity 4,096    4.7 / 5.7 / 7.2 / 7.4 / 8.1 / 10.1 / 13.3
+//               capacity 8,192    4.6 / 5.6 / 7.2 / 8.1 / 8.6 /  9.9 / 12.0 / 16.2
+//   two launches, 1,024           6.3 / 7.2 / 8.1 / 8.4 / 9.6
+//                 8,192           6.1 / 7.1 / 8.7 / 8.8 / 9.1 / 10.4 / 12.4 / 16.5
+//   one workgroup per head        5.9 / 6.7 / 7.3 / 8.0 / 11.3 / 21.4 / 36.4 / 66
+// Two launches lose to one workgroup per head below ~350 positions (the second launch is 1.4 us that nothing can take
+// back once it is enqueued); only a captured call that holds no workspace takes them. Plans of 512 and 768 workgroups with
+// smaller head groups: up to 0.6 us less at position 100, 3-6 us more at 8,100; groups of up to 8 heads: 2.5 us more at 100.
 constexpr int kAsWorkgroups = 256;
 
 static int attn_least_splits(int max_len) {
@@ -624,8 +663,15 @@ static int attn_least_splits(int max_len) {
 static int attn_head_groups(int n_kv, int grp, int max_len) {
   const int least = attn_least_splits(max_len);
   int gh = 1;
-  while (gh < grp && gh < kAsMaxHeads && n_kv * ((grp + gh - 1) / gh) * least > kAsWorkgroups) ++gh;
+  while (gh < grp && gh < kAsMaxHeads && (int64_t)n_kv * ((grp + gh - 1) / gh) * least > kAsWorkgroups) ++gh;
   return (grp + gh - 1) / gh;
+}
+
+// Passes up to which a workgroup per head holds all positions (no merge) in a plan of GH heads per workgroup: a pass costs
+// 0.85 us, spreading the passes costs the merge and GH heads' work per workgroup. Without counters the merge is a launch
+// that is there in any case, so less is saved.
+static int attn_direct_passes(int slots, bool counters) {
+  return slots <= 2 ? 3 : std::min(slots + 1, counters ? 6 : 4);
 }
 
 // (at least a pass of 64 positions each)
@@ -680,19 +726,23 @@ extern "C" int exl3_attn_decode_rotate_ws(const uint16_t* q, const uint16_t* k, 
                  workspace_bytes);
     const int grp = n_heads / n_kv_heads, z = attn_head_groups(n_kv_heads, grp, max_len), gh = (grp + z - 1) / z;
     const int splits = attn_splits(n_kv_heads, z, max_len);
-    const int passes = (max_len + splits * kAsPass - 1) / (splits * kAsPass);
+    const int slots = gh <= 4 ? gh : gh <= 6 ? 6 : 8;   // heads the kernel is built for
+    // (a workgroup of the head group for each of its heads)
+    const int direct_passes = std::min(slots, grp) <= splits ? attn_direct_passes(slots, counters != nullptr) : 0;
+    const int passes = std::max((max_len + splits * kAsPass - 1) / (splits * kAsPass), direct_passes);
     float* part_o = static_cast<float*>(workspace);
-    const AttnSplitArgs a{q, k, v, k_cache, v_cache, pos, rope_cos, rope_sin, grp, max_len, splits, passes, scale, part_o,
+    const AttnSplitArgs a{q, k, v, k_cache, v_cache, pos, rope_cos, rope_sin, grp, max_len, splits, passes, direct_passes * kAsPass, scale,
+                          part_o,
                           reinterpret_cast<float2*>(part_o + (size_t)n_heads * splits * kAttnHD), counters, suh, o, xh};
     const dim3 grid((unsigned)splits, (unsigned)n_kv_heads, (unsigned)z);
-    if (gh <= 1) launch_attn_split<1>(grid, a, st);
-    else if (gh <= 2) launch_attn_split<2>(grid, a, st);
-    else if (gh <= 3) launch_attn_split<3>(grid, a, st);
-    else if (gh <= 4) launch_attn_split<4>(grid, a, st);
-    else if (gh <= 6) launch_attn_split<6>(grid, a, st);
+    if (slots == 1) launch_attn_split<1>(grid, a, st);
+    else if (slots == 2) launch_attn_split<2>(grid, a, st);
+    else if (slots == 3) launch_attn_split<3>(grid, a, st);
+    else if (slots == 4) launch_attn_split<4>(grid, a, st);
+    else if (slots == 6) launch_attn_split<6>(grid, a, st);
     else launch_attn_split<8>(grid, a, st);
     if (!counters)
-      attn_merge_kernel<<<n_heads, kAmThreads, 0, st>>>(a.part_o, a.part_ml, pos, max_len, splits, suh, o, xh);
+      attn_merge_kernel<<<n_heads, kAmThreads, 0, st>>>(a.part_o, a.part_ml, pos, max_len, a.direct, splits, suh, o, xh);
     EXL3_LAUNCH_CHECK("exl3_attn_decode_rotate_ws");
     return EXL3_OK;
   }

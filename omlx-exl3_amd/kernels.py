@@ -11,8 +11,11 @@ kernels.py:269-270, 465); the C library re-validates and its status becomes an E
 """
 from __future__ import annotations
 
+import collections
 import ctypes
+import functools
 import math
+import threading
 
 import torch
 
@@ -539,7 +542,7 @@ def prefill_gemm(xh: torch.Tensor, trellis: torch.Tensor, k: int, n: int, K: int
 
 
 # Decode attention by cache capacity: one workgroup per head up to the first bound; above it the positions are split
-# over workgroups, merged by the last to arrive when the caller holds an attn_workspace, else by a second launch
+# over workgroups, merged by the last to arrive where a workspace is held, else by a second launch
 # (exl3_attn_decode_rotate_ws; measured sides at csrc/exl3_attn.hip's plan).
 ATTN_UNSPLIT_LEN = 512
 ATTN_MAX_LEN = 8192
@@ -555,13 +558,50 @@ def attn_workspace(n_heads: int, n_kv: int, max_len: int, device) -> torch.Tenso
     return torch.zeros(256 * n_heads + nbytes, dtype=torch.uint8, device=device)
 
 
+@functools.lru_cache(maxsize=256)
+def _attn_workspace_bytes(n_heads: int, n_kv: int, max_len: int) -> int:
+    return lib().exl3_attn_decode_workspace_bytes(n_heads, n_kv, max_len)
+
+
+class _AttnScratch(threading.local):
+    """attn_workspace of the shapes and streams a thread last called attn_decode_rotate with while it held none: calls on
+    a stream follow each other, so one workspace per (stream, shape) serves them, and a thread shares its own with no
+    other. At most 8 of at most 2 MiB each, the least recently used given back; all are at the thread's end."""
+
+    ENTRIES, ENTRY_BYTES = 8, 2 << 20
+
+    def __init__(self):
+        self.held = collections.OrderedDict()
+
+    def get(self, n_heads: int, n_kv: int, max_len: int, device: torch.device, stream: int) -> torch.Tensor | None:
+        """The workspace, or None where none may be held: a capture's launches run again at any time, on any stream."""
+        if device.index != torch.cuda.current_device() or torch.cuda.is_current_stream_capturing():
+            return None
+        key = (device.index, stream, n_heads, n_kv, max_len)
+        ws = self.held.get(key)
+        if ws is None:
+            if 256 * n_heads + _attn_workspace_bytes(n_heads, n_kv, max_len) > self.ENTRY_BYTES:
+                return None
+            ws = self.held[key] = attn_workspace(n_heads, n_kv, max_len, device)
+            if len(self.held) > self.ENTRIES:
+                self.held.popitem(last=False)
+        else:
+            self.held.move_to_end(key)
+        return ws
+
+
+_attn_scratch = _AttnScratch()
+
+
 def attn_decode_rotate(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cache: torch.Tensor,
                        v_cache: torch.Tensor, pos: torch.Tensor, rope_cos: torch.Tensor, rope_sin: torch.Tensor,
                        suh: torch.Tensor | None, want_o: bool = False, workspace: torch.Tensor | None = None):
     """Batch-1 decode attention with rotary embedding and KV-cache append, producing o_proj's rotated input
     (exl3_attn_decode_rotate). q (n_heads*128,), k / v (n_kv*128,) fp16 (views of one row are fine);
     caches fp16 (n_kv, max_len, 128); pos int64 (1,) on the device; rope tables fp32 (max_len, 64).
-    workspace: attn_workspace of this shape, held by the caller, or None (one is allocated where it is needed).
+    workspace: attn_workspace of this shape, held by the caller, or None: an eager call then takes one kept for its thread,
+    stream and shape (_AttnScratch); a captured call allocates the sums' memory and merges in a second launch (~1.4 us
+    more per replay), so a program that captures its decode step holds one.
     Returns (xh (1, 1, n_heads*128) or None, o (1, n_heads*128) or None)."""
     for t, name in ((k_cache, "k_cache"), (v_cache, "v_cache"), (rope_cos, "rope_cos"), (rope_sin, "rope_sin")):
         _dev(t, name)
@@ -585,18 +625,21 @@ def attn_decode_rotate(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, k_cach
     if max_len <= ATTN_UNSPLIT_LEN or max_len > ATTN_MAX_LEN:      # (the entry point refuses what is too long)
         check(lib().exl3_attn_decode_rotate(*args, stream_handle(q.device)), "exl3_attn_decode_rotate")
         return xh, o
-    nbytes = lib().exl3_attn_decode_workspace_bytes(n_heads, n_kv, max_len)
-    if workspace is not None:
+    nbytes = _attn_workspace_bytes(n_heads, n_kv, max_len)
+    stream = stream_handle(q.device)
+    if workspace is None:
+        workspace = _attn_scratch.get(n_heads, n_kv, max_len, q.device, stream)
+    else:
         _dev(workspace, "workspace")
         _require(workspace.dtype == torch.uint8 and workspace.numel() == 256 * n_heads + nbytes,
                  "attn_decode_rotate: workspace is attn_workspace of this shape")
+    if workspace is not None:
         counters = workspace.data_ptr()
         ws = counters + 256 * n_heads
     else:
         buf = torch.empty(nbytes, dtype=torch.uint8, device=q.device)
         counters, ws = None, buf.data_ptr()
-    check(lib().exl3_attn_decode_rotate_ws(*args, ws, nbytes, counters, stream_handle(q.device)),
-          "exl3_attn_decode_rotate")
+    check(lib().exl3_attn_decode_rotate_ws(*args, ws, nbytes, counters, stream), "exl3_attn_decode_rotate")
     return xh, o
 
 
