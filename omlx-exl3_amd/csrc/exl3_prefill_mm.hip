@@ -376,43 +376,89 @@ __global__ __launch_bounds__(kMmThreads) __attribute__((amdgpu_waves_per_eu(2)))
 }
 
 // Launch plan of a shape (from rows, k and n only): tile height (64 ti rows) and a split of k over S workgroups per
-// tile, the pair of least estimated time. A round of w workgroups (256 at most, one per CU) takes, per 64-k step of a
-// split, a[ti] + b[ti] w / 256 us (the more CUs work, the lower the clock), and f[ti] besides; S > 1 adds the reduction
-// launch: 1.2 + 0.31 S us and S + 1 passes over an fp32 rows x n array at 3.16 TB/s (2.3 TB/s beyond 48 MB), and a
-// workspace of S x rows x n fp32, held to kPrefillWorkspaceLimit. At least 4 steps per split, S <= 16. The constants were
-// fitted to 111 shapes (k 1,024-17,408, n 512-17,408, 200-4,608 rows) x 3 heights x up to 8 splits, over which the pick
-// is on average within 2% of the fastest measured pair (4% for the rule before, which picked the height first and split
-// launches of at most 128 tiles). The sides, us before / now: 17408 -> 5120 at 777 / 1,024 / 1,300 rows 218 / 233 / 234
-// against 153 / 166 / 215; 5120 -> 1024 at 777 / 1,024 rows 28.5 / 33.5 against 22.9 / 24.4; 8192 -> 1024 at 3,000 rows 70
-// against 59; the largest loss, 5120 -> 1024 at 1,300 rows, 28.2 against 29.6.
+// tile, S > 1 with a workspace of S x rows x n fp32, held to kPrefillWorkspaceLimit.
+//
+// Two rules. mm_round_plan: the height with the fewest rounds of 256 workgroups times rows of a tile, then, where that
+// leaves at most 128 tiles, the S of least rounds x steps. mm_us: an estimate of the time of any pair, fitted to 456 shapes
+// (k 512-17,408, n 512-17,408, 129-8,192 rows, whole calls from graphs) x 3 heights x up to 11 splits. The pair of least
+// estimated time is taken where it is ahead of the round plan's by 0.7 us + 2%, by a third of that for another S of its
+// height where it splits already: what the estimate does not see (caches, the order of tiles) costs as much. On 653 shapes,
+// 197 of them not fitted to, calls are 0.9% faster on average than by the round plan, 15 of them more than 2% slower than
+// by it (by an estimate alone, of earlier constants: 0.3%, 65 of them, 2048 -> 3072 at 777 rows 34.6 -> 40.1 us, 10496 ->
+// 1536 at 4,098 rows 158 -> 177). Whole calls, round plan / now: 17408 -> 5120 at 777 /
+// 1,024 / 1,536 rows 201 / 216 / 284 against 195 / 203 / 268; 8192 -> 1024 at 3,000 rows 76.6 against 65.3; 5120 -> 1024 at
+// 1,024 rows 33.8 against 30.0.
 struct MmPlan {
   int ti, tiles_m, splits, steps_per_split;
 };
 
-static MmPlan mm_plan(int rows, int k, int n) {
-  static const double a[3] = {0.575, 0.603, 0.770}, b[3] = {0.270, 0.392, 0.452}, f[3] = {3.3, 8.2, 8.9};
+// S splits of nsteps 64-k steps without an empty one
+static MmPlan mm_pair(int rows, int nsteps, int ti, int S) {
+  const int sps = (nsteps + S - 1) / S;
+  return MmPlan{ti, (rows + 64 * ti - 1) / (64 * ti), (nsteps + sps - 1) / sps, sps};
+}
+
+// Estimated time (us). A round of w workgroups (256 at most, one per CU) takes, per 64-k step of a split, a + b x + c x^2
+// with x = w / 256, and f besides; S = 1 adds the epilogue, e (1 + 2.3 x), to each round, S > 1 the reduction launch: 2.13
+// us and S + 1 passes over an fp32 rows x n array at 2.4 TB/s up to 14 MB in all, 4.8 TB/s beyond.
+static double mm_us(const MmPlan& p, int rows, int n) {
+  static const double a[3] = {0.480, 0.683, 0.902}, b[3] = {-0.133, -0.291, -0.443}, c[3] = {0.211, 0.360, 0.497}, f[3] = {2.41, 3.23, 4.25}, e[3] = {3.19, 4.65, 6.02};
+  const long groups = (long)p.tiles_m * ((n + kMmBN - 1) / kMmBN) * p.splits;
+  const int i = p.ti - 2;
+  auto round_us = [&](long w) {
+    const double x = (double)w / 256.0;
+    return p.steps_per_split * (a[i] + (b[i] + c[i] * x) * x) + f[i] + (p.splits == 1 ? e[i] * (1.0 + 2.3 * x) : 0.0);
+  };
+  double us = (double)(groups / 256) * round_us(256) + (groups % 256 ? round_us(groups % 256) : 0.0);
+  if (p.splits > 1) {
+    const double mb = (p.splits + 1) * ((double)rows * n * 4e-6);
+    us += 2.13 + 0.42 * mb - (mb > 14.0 ? 0.214 * (mb - 14.0) : 0.0);
+  }
+  return us;
+}
+
+static MmPlan mm_round_plan(int rows, int k, int n) {
   const int nsteps = k / kMmBK;
   const long tiles_n = (n + kMmBN - 1) / kMmBN;
-  const double out_bytes = (double)rows * n * 4.0;
-  MmPlan best{};
-  double best_us = -1.0;
+  auto tiles = [&](int ti) { return (long)((rows + 64 * ti - 1) / (64 * ti)) * tiles_n; };
+  int ti = 4;
+  for (int t = 3; t >= 2; --t)
+    if ((tiles(t) + 255) / 256 * (t + 1) < (tiles(ti) + 255) / 256 * (ti + 1)) ti = t;
+  int best = 1;
+  if (tiles(ti) <= 128) {
+    const double step_us = 0.55 * ti, pass_us = (double)rows * n * 1e-6;
+    double best_us = nsteps * step_us;
+    for (int S = 2; S <= 16; ++S) {
+      const int sps = (nsteps + S - 1) / S;
+      if (sps < 4 || (size_t)S * rows * n * sizeof(float) > kPrefillWorkspaceLimit) break;
+      const double us = (double)((tiles(ti) * S + 255) / 256) * sps * step_us + (S + 1) * pass_us + 3.0;
+      if (us < best_us) {
+        best = S;
+        best_us = us;
+      }
+    }
+  }
+  return mm_pair(rows, nsteps, ti, best);
+}
+
+static MmPlan mm_plan(int rows, int k, int n) {
+  const int nsteps = k / kMmBK;
+  const MmPlan round = mm_round_plan(rows, k, n);
+  MmPlan best = round;
+  double best_us = mm_us(round, rows, n);
+  const double margin_us = 0.7 + 0.02 * best_us;
   for (int ti = 4; ti >= 2; --ti) {
     if (ti > 2 && rows <= 64 * (ti - 1)) continue;   // one tile row of a smaller height holds them
-    const int tiles_m = (rows + 64 * ti - 1) / (64 * ti);
-    const long tiles = (long)tiles_m * tiles_n;
     for (int S = 1; S <= 16; ++S) {
-      const int sps = (nsteps + S - 1) / S;
-      if (S > 1 && (sps < 4 || tiles * S > 1024 || S * out_bytes > (double)kPrefillWorkspaceLimit)) break;
-      if ((nsteps + sps - 1) / sps != S) continue;   // an S that leaves an empty split: the plan of a smaller one
-      const long groups = tiles * S, rest = groups % 256;
-      auto round_us = [&](long w) { return sps * (a[ti - 2] + b[ti - 2] * (double)w / 256.0) + f[ti - 2]; };
-      double us = (double)(groups / 256) * round_us(256) + (rest ? round_us(rest) : 0.0);
-      if (S > 1) {
-        const double bytes = (S + 1) * out_bytes;
-        us += 1.2 + 0.31 * S + bytes / 3.16e6 + (bytes > 48e6 ? (bytes - 48e6) / 8.46e6 : 0.0);
-      }
-      if (best_us < 0 || us < best_us) {
-        best = MmPlan{ti, tiles_m, S, sps};
+      const MmPlan p = mm_pair(rows, nsteps, ti, S);
+      if (S > 1 && (p.steps_per_split < 4 || (long)p.tiles_m * ((n + kMmBN - 1) / kMmBN) * S > 1024 ||
+                    (size_t)S * rows * n * sizeof(float) > kPrefillWorkspaceLimit))
+        break;
+      if (p.splits != S) continue;   // an S that leaves a split empty: the plan of a smaller one
+      const bool near = ti == round.ti && S > 1 && round.splits > 1;
+      const double us = mm_us(p, rows, n) + (near ? 0.3 : 1.0) * margin_us;
+      if (us < best_us) {
+        best = p;
         best_us = us;
       }
     }

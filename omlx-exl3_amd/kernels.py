@@ -386,6 +386,17 @@ class TrellisGemvPlan:
         return out
 
 
+# (pure functions of the shape; planning one takes longer than looking it up)
+@functools.lru_cache(maxsize=1024)
+def _matmul_workspace_bytes(rows: int, k: int, n: int, n_call: int) -> int:
+    return lib().exl3_prefill_matmul_window_workspace_bytes(rows, k, n, n_call)
+
+
+@functools.lru_cache(maxsize=1024)
+def _rows_workspace_bytes(rows: int, k: int, n: int, K: int, splits: int) -> int:
+    return lib().exl3_prefill_rows_workspace_bytes(rows, k, n, K, splits)
+
+
 def prefill_matmul(xh: torch.Tensor, wt: torch.Tensor, svh: torch.Tensor, bias: torch.Tensor | None,
                    out: torch.Tensor, n_call: int | None = None) -> torch.Tensor:
     """had128(xh @ wt^T) * svh (+ bias) into out by the hand-written MFMA GEMM (exl3_prefill_matmul): xh (rows, k)
@@ -405,7 +416,7 @@ def prefill_matmul(xh: torch.Tensor, wt: torch.Tensor, svh: torch.Tensor, bias: 
              "prefill_matmul: out must be (rows, n) with unit column stride")
     ldy = out.stride(0) if rows > 1 else n
     n_call = n if n_call is None else n_call
-    nbytes = lib().exl3_prefill_matmul_window_workspace_bytes(rows, k, n, n_call)
+    nbytes = _matmul_workspace_bytes(rows, k, n, n_call)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=xh.device) if nbytes else None
     check(lib().exl3_prefill_matmul_window(ptr(xh), ptr(wt), rows, k, n, n_call, ptr(svh), ptr(bias), ptr(out), ldy,
                                            DTYPE_CODE[out.dtype], ptr(ws), nbytes, stream_handle(xh.device)),
@@ -431,7 +442,7 @@ def prefill_rows(xh: torch.Tensor, trellis: torch.Tensor, k: int, n: int, K: int
 
 def _prefill_rows(xh, trellis, k, n, K, cb, svh, bias, out, rows, splits):
     """prefill_rows' launch, its arguments checked by the caller."""
-    nbytes = lib().exl3_prefill_rows_workspace_bytes(rows, k, n, K, splits)
+    nbytes = _rows_workspace_bytes(rows, k, n, K, splits)
     ws = torch.empty(nbytes, dtype=torch.uint8, device=xh.device) if nbytes else None
     check(lib().exl3_prefill_rows(ptr(xh), ptr(trellis), k, n, K, cb, ptr(svh), ptr(bias), ptr(out),
                                   DTYPE_CODE[out.dtype], rows, splits, ptr(ws), nbytes, stream_handle(xh.device)),
@@ -530,10 +541,12 @@ def prefill_gemm(xh: torch.Tensor, trellis: torch.Tensor, k: int, n: int, K: int
         y2 = out.view(rows, n)
         wt = torch.empty((chunks[0][1], k), dtype=torch.float16, device=xh.device)
         for c0, cn in chunks:
-            w = wt[:cn]
-            check(lib().exl3_reconstruct(ptr(trellis), k, n, K, cb, c0 // 16, cn // 16, ptr(w),
+            check(lib().exl3_reconstruct(ptr(trellis), k, n, K, cb, c0 // 16, cn // 16, ptr(wt),
                                          stream_handle(xh.device)), "exl3_reconstruct")
-            prefill_matmul(x2, w, svh[c0:c0 + cn], None if bias is None else bias[c0:c0 + cn], y2[:, c0:c0 + cn],
+            if cn == n:      # (the whole call: no views)
+                prefill_matmul(x2, wt, svh, bias, y2)
+                break
+            prefill_matmul(x2, wt[:cn], svh[c0:c0 + cn], None if bias is None else bias[c0:c0 + cn], y2[:, c0:c0 + cn],
                            n_call=n)
         return out
     check(lib().exl3_prefill_gemm(ptr(xh), ptr(trellis), k, n, K, cb, ptr(svh), ptr(bias), ptr(out),

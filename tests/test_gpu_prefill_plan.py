@@ -33,12 +33,13 @@ def _operands(rows, k, n):
             torch.randn(n, device="cuda", generator=g) * 0.1)
 
 
-# (tile height, splits): 256 rows x 3 and x 2, 192 x 4, 128 x 5, 128 x 8 with a ragged last split; rows and n ragged too
-@pytest.mark.parametrize("rows,k,n,splits", [(777, 17408, 5120, 3), (1300, 17408, 5120, 2), (3000, 8192, 1024, 4),
-                                             (1000, 5120, 1152, 5), (641, 5184, 640, 0)])
-def test_prefill_matmul_split_plans(pk, rows, k, n, splits):
+# shapes that split k, at tile heights of 256, 192 and 128 rows when this was written (the plan may be fitted anew): even
+# and ragged splits, ragged rows and columns
+@pytest.mark.parametrize("rows,k,n", [(777, 17408, 5120), (1536, 17408, 5120), (3000, 8192, 1024), (1000, 5120, 1152),
+                                      (641, 5184, 640)])
+def test_prefill_matmul_split_plans(pk, rows, k, n):
     nbytes = pk._capi.lib().exl3_prefill_matmul_workspace_bytes(rows, k, n)
-    assert nbytes % (rows * n * 4) == 0 and (not splits or nbytes // (rows * n * 4) == splits)
+    assert nbytes > 0 and nbytes % (rows * n * 4) == 0
     xh, wt, svh, bias = _operands(rows, k, n)
     for dt, bar in ((torch.float16, 2e-3), (torch.float32, 2e-3)):
         b = bias.to(dt)
