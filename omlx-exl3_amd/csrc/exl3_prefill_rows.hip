@@ -10,12 +10,14 @@
 
 namespace exl3 {
 
-// Launch plan, from rows, k and n only: row blocks of up to 256 rows (16 RT), and S splits of k. The time of a plan is
+// Launch plan, from rows, k, n and K only: row blocks of up to 256 rows (16 RT), and S splits of k. The time of a plan is
 // estimated from what was measured at 7 shapes (k 1,024-17,408, n 1,024-17,408) x 15 row counts x up to 13 splits: a
 // 64-k step of a workgroup costs 0.195 + 0.0355 RT us when others share its CU, at least 0.21 + 0.055 RT alone (latency),
-// kRowsResident workgroups fit a CU, ~6.3 us are fixed, and the splits' sums are written and read once at ~6.4 TB/s
-// plus a second launch. Automatic plans split while the sums stay within kPrefillWorkspaceLimit (a wide head has column
-// blocks enough: 92 rows of 17408 -> 151936 took 160 MiB of sums, 246 rows 428 MiB). Over those shapes the pick is within 4% of the best measured plan except at a few small ones.
+// two to four workgroups fit a CU, ~6.3 us are fixed, and the splits' sums are written and read once at ~6.4 TB/s
+// plus a second launch. Over 500 other shapes (150-1,100 rows, 2-8 bits) the pick's S is 0.7% behind the best measured one
+// on average, 49 of them more than 3% (14% at most). Automatic plans split while the sums stay within
+// kPrefillWorkspaceLimit (a wide head has column blocks enough: 92 rows of 17408 -> 151936 took 160 MiB of sums, 246 rows
+// 428 MiB).
 struct RowsPlan {
   int rt, row_blocks, splits, kt_per_split;
 };
@@ -25,8 +27,8 @@ static int rows_rt(int rows) {   // the smallest built tile count that holds the
   return tiles <= 4 ? tiles : tiles <= 6 ? 6 : tiles <= 8 ? 8 : tiles <= 12 ? 12 : 16;
 }
 
-static double rows_cost(int rt, long groups, int steps_per_split, int splits, double out_bytes) {
-  const int resident = rt <= 6 ? 4 : rt <= 12 ? 3 : 2;
+static double rows_cost(int K, int rt, long groups, int steps_per_split, int splits, double out_bytes) {
+  const int resident = rt <= 6 ? 4 : rt <= 8 || (rt <= 12 && K < 8) ? 3 : 2;   // workgroups a CU holds (registers)
   const long per_cu = (groups * splits + 255) / 256;
   const double shared = 0.195 + 0.0355 * rt, alone = 0.21 + 0.055 * rt;
   auto round_us = [&](long g) { return g * shared > alone ? g * shared : alone; };
@@ -35,7 +37,7 @@ static double rows_cost(int rt, long groups, int steps_per_split, int splits, do
   return us + (splits > 1 ? 1.9 + 0.1 * splits + (2 * splits + 0.5) * out_bytes / 6.4e6 : 0.13 * rt);
 }
 
-static RowsPlan rows_plan(int rows, int k, int n, int splits) {
+static RowsPlan rows_plan(int rows, int k, int n, int K, int splits) {
   constexpr int kMaxSplits = 16, kMaxRowsPerBlock = 256;
   const int steps = k / 64, z0 = (rows + kMaxRowsPerBlock - 1) / kMaxRowsPerBlock;
   RowsPlan best{};
@@ -52,7 +54,7 @@ static RowsPlan rows_plan(int rows, int k, int n, int splits) {
           (per < 3 || (size_t)S * (size_t)rows * (size_t)n * sizeof(float) > kPrefillWorkspaceLimit))
         break;
       const int real = (steps + per - 1) / per;   // no empty split
-      const double us = rows_cost(rt, (long)(n / 128) * z, per, real, (double)rows * n * 4.0);
+      const double us = rows_cost(K, rt, (long)(n / 128) * z, per, real, (double)rows * n * 4.0);
       if (best_us < 0 || us < best_us) {
         best = RowsPlan{rt, z, real, 4 * per};
         best_us = us;
@@ -82,7 +84,7 @@ static bool rows_shape_ok(int rows, int k, int n, int K) {
 
 extern "C" size_t exl3_prefill_rows_workspace_bytes(int rows, int k, int n, int K, int splits) {
   if (!rows_shape_ok(rows, k, n, K) || !rows_fits(rows, k, n, K) || rows > 65535) return 0;
-  return rows_workspace(rows_plan(rows, k, n, splits), rows, n);
+  return rows_workspace(rows_plan(rows, k, n, K, splits), rows, n);
 }
 
 extern "C" int exl3_prefill_rows(const uint16_t* xh, const uint32_t* trellis, int k, int n, int K, int cb,
@@ -100,7 +102,7 @@ extern "C" int exl3_prefill_rows(const uint16_t* xh, const uint32_t* trellis, in
                "exl3_prefill_rows: xh and y must be 16-byte and trellis 4-byte aligned");
   EXL3_REQUIRE(rows_fits(rows, k, n, K), EXL3_ERR_ARG,
                "exl3_prefill_rows: activations, a split's sums or the trellis exceed 2 GiB");
-  const RowsPlan p = rows_plan(rows, k, n, splits);
+  const RowsPlan p = rows_plan(rows, k, n, K, splits);
   EXL3_REQUIRE(p.splits >= 1 && (p.splits - 1) * p.kt_per_split < k / 16, EXL3_ERR_ARG,
                "exl3_prefill_rows: %d splits leave an empty split", p.splits);
   const size_t need = rows_workspace(p, rows, n);

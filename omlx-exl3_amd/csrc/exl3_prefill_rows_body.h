@@ -245,7 +245,8 @@ __device__ __forceinline__ void rows_body(const RowsArgs& a, u32x4* sA0, u32x4* 
   });
 }
 
-// one kernel per number of 16-row tiles: the LDS stages' size is spelled out (an LDS array whose size depends on a
+// one kernel per number of 16-row tiles, compiled for as many wavefronts per SIMD as its registers allow (RT = 12 at K = 8
+// needs 178, 10 more than three leave: spilled, it took 15-20% longer than reconstruction + GEMM): the LDS stages' size is spelled out (an LDS array whose size depends on a
 // template parameter makes hipcc drop the kernel's host stub when the buffer-to-LDS load builtin writes into it)
 #define EXL3_ROWS_KERNEL(RT, WPE, SLOTS)                                                                         \
   template <int K, int CB>                                                                                       \
@@ -261,7 +262,7 @@ EXL3_ROWS_KERNEL(3, 4, 512)
 EXL3_ROWS_KERNEL(4, 4, 512)
 EXL3_ROWS_KERNEL(6, 4, 768)
 EXL3_ROWS_KERNEL(8, 3, 1024)
-EXL3_ROWS_KERNEL(12, 3, 1536)
+EXL3_ROWS_KERNEL(12, (K == 8 ? 2 : 3), 1536)
 EXL3_ROWS_KERNEL(16, 2, 2048)
 #undef EXL3_ROWS_KERNEL
 
