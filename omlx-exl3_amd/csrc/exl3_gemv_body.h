@@ -78,13 +78,9 @@ __device__ void stage_prologue(const GemvArgs& a, int m, int blk_in_member, int 
     const int kt = c0 >> 4;
     const bool in_split = kt >= kt0 && kt < kt1;
     float v[8];
-    if (a.pro == kProRotB16) {
-      load8<kBF16>(a.px, (size_t)r * k + c0, v);
-    } else {
-      load8<kF16>(a.px, (a.pro == kProSwiglu ? (size_t)r * 2 * k : (size_t)r * k) + c0, v);
-    }
     if (a.pro == kProNorm) {
       float wv[8];
+      load8<kF16>(a.px, (size_t)r * k + c0, v);
       if (a.pres) {
         float rv[8];
         load8<kF16>(a.pres, (size_t)r * k + c0, rv);
@@ -97,8 +93,13 @@ __device__ void stage_prologue(const GemvArgs& a, int m, int blk_in_member, int 
 #pragma unroll
       for (int i = 0; i < 8; ++i) v[i] = round_through<kF16>(wv[i] * round_through<kF16>(v[i] * inv));
       if (write_xn && in_split) store8<kF16>(a.pxn_out, (size_t)r * k + c0, v);
-    } else if (a.pro == kProSwiglu) {
+    } else if (a.pro == kProRot) {
+      load8<kF16>(a.px, (size_t)r * k + c0, v);
+    } else if (a.pro == kProRotB16) {
+      load8<kBF16>(a.px, (size_t)r * k + c0, v);
+    } else {
       float uv[8];
+      load8<kF16>(a.px, (size_t)r * 2 * k + c0, v);
       load8<kF16>(a.px, (size_t)r * 2 * k + k + c0, uv);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
