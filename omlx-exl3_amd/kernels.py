@@ -25,14 +25,15 @@ PROLOGUE_NONE, PROLOGUE_RMSNORM, PROLOGUE_SWIGLU, PROLOGUE_ROTATE = 0, 1, 2, 3  
 MAX_GEMV_ROWS = 8           # rows at or below which EXL3Linear takes the GEMV path (kernels.py:260)
 GEMV_ROWS_LIMIT = 16        # rows one GEMV launch accepts
 GEMV_EXACT, GEMV_FAST, GEMV_TABLE = 0, 1, 2
-# Elements a GEMV launch of several rows rotates inside (every 128-column block rotates its rows again) up to which that
-# beats a rotation launch of its own (~2 us). Measured us, inside / own launch: 6144 -> 5120, 8 rows (2.0 M) 12.5 / 13.9;
-# 5120 -> 2 x 17408, 4 rows (5.6 M) 39.8 / 40.6, 8 rows (11 M) 42.8 / 41.7; 17408 -> 5120, 4 rows (2.8 M) 18.6 / 19.3,
-# 8 rows (5.6 M) 20.8 / 20.4; 5120 -> 151936, 2 / 4 / 8 rows (12 / 24 / 49 M) 134 / 144 / 162 against 130 / 135 / 144. A
-# single row's operands are loaded ahead of the trellis: inside at every shape (5120 -> 151936 129.5 / 133.5).
-# The limit lies above the level pair of 17408 -> 5120: a call that launches twice also takes the host longer than a
-# 20 us launch takes the GPU (3-bit, 8 rows, a call among others: 21.1 us inside, 25.1 with a launch of its own).
-ROTATE_IN_LAUNCH_LIMIT = 8_000_000
+# Where a GEMV launch of several rows rotates its input inside (every 128-column block rotates its rows again, rows * k *
+# n / 128 elements in all) and where a rotation launch of its own (~2 us) comes first. Measured on MI355X over 130 random
+# layers (k 1,024-17,408, n 512-151,936, 2-8 rows, 2-8 bits, fp16 and bf16), GPU time with a launch of its own over inside:
+# 1.00-1.10 to 3 M elements, 0.96-1.02 at 4 M, 0.93-0.99 at 5-6 M, 0.91-0.97 at 8 M. A call that launches twice takes the
+# host ~20 us, what the GPU takes for 80 M weights at these rows: smaller layers rotate inside whatever the elements (14592
+# -> 4736, 8 rows, 4.3 M elements: a call among others 17.6 us inside, 20.5 with two launches; 2304 -> 36736, 8 rows, 5.3 M:
+# 22.4 / 21.1). A single row's operands are loaded ahead of the trellis: inside at every shape (5120 -> 151936 129.5 / 133.5).
+ROTATE_IN_LAUNCH_LIMIT = 4_250_000
+ROTATE_IN_LAUNCH_WEIGHTS = 80_000_000
 
 
 def _require(cond: bool, msg: str) -> None:
@@ -231,7 +232,8 @@ class TrellisGemvPlan:
             nbytes = max(nbytes, self.n // 128 * 256 + (S * rows * self.n * 4 if S > 1 else 0))
         self.workspace = torch.zeros(max(nbytes, 256), dtype=torch.uint8, device=self.device)
         self._ns_c = (ctypes.c_int * 3)(*(list(member_ns) + [0] * (3 - len(member_ns))))
-        self.rotates_inside = rows == 1 or rows * k * (self.n // 128) <= ROTATE_IN_LAUNCH_LIMIT
+        self.rotates_inside = rows == 1 or rows * k * (self.n // 128) <= ROTATE_IN_LAUNCH_LIMIT or \
+            k * self.n < ROTATE_IN_LAUNCH_WEIGHTS
         self._tr_key = None
         self._tr_c = None
 

@@ -65,3 +65,17 @@ def test_linear_on_both_sides_of_the_rotation_rule(pk, rows, inside):
     y = lin(x)
     lin.arm_residual(res)
     assert torch.equal(lin(x), (y.float() + res.float()).half()) and lin.take_armed_output() is not None
+
+
+@pytest.mark.parametrize("k,n,rows,inside", [(14592, 4736, 8, True), (5120, 15616, 8, True), (5120, 15744, 8, False),
+                                             (2304, 36736, 8, False), (1664, 98432, 2, True), (1664, 98432, 4, False)])
+def test_rotation_rule_by_elements_and_weights(pk, k, n, rows, inside):
+    """Up to 4.25 M rotated elements or below 80 M weights the rotation is inside the launch; the bits are the same."""
+    assert inside == (rows * k * n // 128 <= 4_250_000 or k * n < 80_000_000)
+    syn = importlib.import_module(pk.__name__ + ".synthetic")
+    g = torch.Generator(device="cuda").manual_seed(n)
+    lin = syn.random_exl3_linear(k, n, 2, 0, g, "cuda")
+    for dt in (torch.float16, torch.bfloat16):
+        x = torch.randn(rows, k, device="cuda", generator=g).to(dt)
+        assert lin._plan(rows, dt).rotates_inside == inside
+        assert torch.equal(lin(x), lin.gemv_rotated(pk.kernels.rot(x, lin.rot_suh), dt))
