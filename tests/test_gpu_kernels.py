@@ -426,7 +426,7 @@ def test_prefill_output_head_in_bounded_windows(pk):
     torch.cuda.synchronize()
     torch.cuda.reset_peak_memory_stats()
     base = torch.cuda.memory_allocated()
-    F.prefill_gemm(xh, tr, k, n, K, 0, svh, out_dtype=torch.float32, out=out)
+    F.prefill_gemm(xh, tr, k, n, K, 0, svh, out_dtype=torch.float32, out=out, path="matmul")
     torch.cuda.synchronize()
     transient = torch.cuda.max_memory_allocated() - base
     assert transient <= chunks[0][1] * k * 2 + (64 << 20), transient

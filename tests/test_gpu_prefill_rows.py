@@ -113,3 +113,35 @@ def test_group_prefill_equals_its_members(pk, rows, dt):
     hook.remove()
     with pytest.raises(ValueError):
         group(x.reshape(-1, 512))
+
+
+@pytest.mark.parametrize("rows", [33, 246])
+def test_prefill_rows_output_head(pk, rows):
+    """The 27B output head, 5120 -> 151936 at K = 6, through the default form of few rows: one launch over all columns,
+    against the fp32 product of decode_wt's weights (bar 2e-3), its transient memory the splits' sums alone (128 MiB at
+    most)."""
+    k, n, K = 5120, 151936, 6
+    F = pk.kernels
+    assert F.takes_rows_form(rows, k, n, K)
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    tr = torch.randint(-32768, 32768, (k // 16, n // 16, 16 * K), dtype=torch.int16, device="cuda", generator=g)
+    svh = (torch.randn(n, device="cuda", generator=g) * 0.01).half()
+    xh = torch.randn((rows, k), device="cuda", generator=g).half()
+    out = torch.empty((rows, n), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    base = torch.cuda.memory_allocated()
+    F.prefill_gemm(xh, tr, k, n, K, 0, svh, out_dtype=torch.float32, out=out)
+    torch.cuda.synchronize()
+    assert torch.cuda.max_memory_allocated() - base <= 128 << 20
+    h = torch.ones(1, 1, device="cuda")
+    for _ in range(7):
+        h = torch.cat((torch.cat((h, h), 1), torch.cat((h, -h), 1)), 0)
+    for c0 in range(0, n, 25344):
+        cn = min(25344, n - c0)
+        W = F.decode_wt(tr, k, n, K, 0, nt0=c0 // 16, ntc=cn // 16).float()
+        y = xh.float() @ W.T
+        del W
+        ref = (y.reshape(-1, 128) @ (h / 128 ** 0.5)).reshape(rows, cn) * svh[c0:c0 + cn].float()
+        err = ((out[:, c0:c0 + cn] - ref).abs().max() / ref.abs().max()).item()
+        assert err < 2e-3, (c0, err)
