@@ -377,9 +377,11 @@ class TrellisGemvPlan:
         """The checks of a call without an epilogue, and its output. A small layer spends longer in its host lines than
         on the GPU, so only what this call can get wrong is looked at (an output made here shares no memory with
         anything): a one-row call of 4096^2 at 4 bits took 18.3 us through fused, and takes 10.0."""
-        if not (x.is_cuda and x.is_contiguous() and x.dtype == dtype and x.numel() == self.rows * self.k):
+        if not (isinstance(x, torch.Tensor) and x.is_cuda and x.is_contiguous() and x.dtype == dtype
+                and x.numel() == self.rows * self.k):
             raise ValueError(f"x must be a contiguous {dtype} tensor ({self.rows}, {self.k}) on the HIP device")
-        if not (suh.is_cuda and suh.is_contiguous() and suh.dtype == torch.float16 and suh.numel() == self.nsub * self.k):
+        if not (isinstance(suh, torch.Tensor) and suh.is_cuda and suh.is_contiguous() and suh.dtype == torch.float16
+                and suh.numel() == self.nsub * self.k):
             raise ValueError("suh must be a contiguous fp16 tensor (n_members, k) on the HIP device")
         given = out is not None
         out = self._bind(trellises, bias, out, x.device)

@@ -79,3 +79,21 @@ def test_rotation_rule_by_elements_and_weights(pk, k, n, rows, inside):
         x = torch.randn(rows, k, device="cuda", generator=g).to(dt)
         assert lin._plan(rows, dt).rotates_inside == inside
         assert torch.equal(lin(x), lin.gemv_rotated(pk.kernels.rot(x, lin.rot_suh), dt))
+
+
+@pytest.mark.parametrize("rows", [1, 3, 16])
+def test_gemv_rotate_fp16_entry(pk, rows):
+    """exl3_gemv_rotate takes fp16 input too (the package calls exl3_gemv_fused for it): the same bits."""
+    k, ns, Ks = 1024, [256, 128], [4, 6]
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    trs = [torch.randint(-32768, 32768, (k // 16, n // 16, 16 * K), dtype=torch.int16, device="cuda", generator=g)
+           for n, K in zip(ns, Ks)]
+    half = lambda *s: torch.randn(s, device="cuda", generator=g).half()
+    plan = pk.kernels.TrellisGemvPlan(k, ns, Ks, 0, half(sum(ns)) / k ** 0.5, rows, torch.float16)
+    x, suh, c = half(rows, k), half(2, k), pk._capi
+    y = plan._rotate_args(x, torch.float16, suh, trs, None, None)
+    c.check(c.lib().exl3_gemv_rotate(c.ptr(x), c.DTYPE_CODE[x.dtype], c.ptr(suh), plan._tr_c, 2, plan._ns_c, plan._Ks_c, k,
+                                     0, c.ptr(plan.svh), None, c.ptr(y), c.DTYPE_CODE[y.dtype], rows,
+                                     c.ptr(plan.workspace), plan.workspace.numel(), c.stream_handle(x.device)),
+            "exl3_gemv_rotate")
+    assert torch.equal(y, plan.rotate(x, suh, trs))

@@ -129,6 +129,15 @@ def test_gemv_plan_member_bitrates():
         kernels.TrellisGemvPlan(256, [128, 128], (4,), 0, svh, 1)
 
 
+@pytest.mark.parametrize("x", [None, np.zeros((1, 256), np.float16), torch.zeros(1, 256, dtype=torch.float16)])
+def test_gemv_plan_rotate_refuses_what_is_no_device_tensor(x):
+    plan = kernels.TrellisGemvPlan(256, [128], 4, 0, torch.ones(128, dtype=torch.float16), 1)
+    tr = torch.zeros(16, 8, 64, dtype=torch.int16)
+    for call in (plan.rotate, plan.rotate_bf16):
+        with pytest.raises(ValueError):
+            call(x, torch.ones(1, 256, dtype=torch.float16), [tr])
+
+
 # ------------------------------------------------------------------------------------------ loader
 class _Attn(nn.Module):
     def __init__(self, h, q, kv):
