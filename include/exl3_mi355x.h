@@ -261,7 +261,8 @@ size_t exl3_prefill_matmul_window_workspace_bytes(int rows, int k, int n, int n_
  *   k % 64 == 0, n % 128 == 0, 1 <= rows <= 65535; activations, trellis and rows x n x 4 bytes each below 2 GiB.
  *   splits: workgroups per (row block, column block) over k, 0 = automatic; more than one needs a 16-byte aligned
  *   workspace of exl3_prefill_rows_workspace_bytes(rows, k, n, K, splits) bytes (uninitialised is fine) and a second
- *   launch that adds the splits' fp32 sums in order. Deterministic; the split depends on the shape only. */
+ *   launch that adds the splits' fp32 sums in order (automatic: at most 128 MiB). Deterministic; the split depends on
+ *   the shape and K only. */
 int exl3_prefill_rows(const uint16_t* xh, const uint32_t* trellis, int k, int n, int K, int cb, const uint16_t* svh,
                       const void* bias, void* y, int out_dtype, int rows, int splits, void* workspace,
                       size_t workspace_bytes, void* stream);
@@ -299,7 +300,8 @@ int exl3_attn_decode_rotate(const uint16_t* q, const uint16_t* k, const uint16_t
                             uint16_t* o, uint16_t* xh, void* stream);
 
 /* exl3_attn_decode_rotate with a workspace: the positions are spread over workgroups, each serving a group of a
- * key/value head's query heads (a cached row is read once per group), and their results merged.
+ * key/value head's query heads (a cached row is read once per group), and their results merged; few positions are held
+ * by one workgroup per head, which writes the outputs itself.
  *   workspace  exl3_attn_decode_workspace_bytes(n_heads, n_kv_heads, max_len) bytes, 16-byte aligned, uninitialised is
  *              fine, not shared by calls in flight together; NULL runs exl3_attn_decode_rotate
  *   counters   NULL: a second launch merges; or n_heads x 256 bytes (uint32 every 64 words) zeroed once before the first

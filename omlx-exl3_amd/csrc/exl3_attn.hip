@@ -643,8 +643,8 @@ static void launch_attn_split(const dim3& grid, const AttnSplitArgs& a, hipStrea
 // workgroup's latency grows with its heads (~0.5 us each) and its passes (at most kAsMaxPasses at full capacity: their
 // scores stay in LDS), so the smallest head groups are taken that leave S that many workgroups; more groups than CUs, or
 // more splits, cost more in dispatch and merge than they save. Measured at 48 / 8 heads, us, graph replays of one call
-// (rows in the caches from the replay before; in a decode step, among the layers' weights, 9.6 at position 700 of 1,024),
-// position 15 / 100 / 200 / 300 / 700 / 2,000 / 4,000 / 8,100:
+// (rows in the caches from the replay before; in a decode step, among the layers' weights, 9.8-10.4 at position 700 of
+// 1,024), position 15 / 100 / 200 / 300 / 700 / 2,000 / 4,000 / 8,100:
 //   one launch, capacity 1,024    4.8 / 5.9 / 7.0 / 7.3 / 8.4
 //               capacity 4,096    4.7 / 5.7 / 7.2 / 7.4 / 8.1 / 10.1 / 13.3
 //               capacity 8,192    4.6 / 5.6 / 7.2 / 8.1 / 8.6 /  9.9 / 12.0 / 16.2
@@ -731,8 +731,8 @@ extern "C" int exl3_attn_decode_rotate_ws(const uint16_t* q, const uint16_t* k, 
     const int direct_passes = std::min(slots, grp) <= splits ? attn_direct_passes(slots, counters != nullptr) : 0;
     const int passes = std::max((max_len + splits * kAsPass - 1) / (splits * kAsPass), direct_passes);
     float* part_o = static_cast<float*>(workspace);
-    const AttnSplitArgs a{q, k, v, k_cache, v_cache, pos, rope_cos, rope_sin, grp, max_len, splits, passes, direct_passes * kAsPass, scale,
-                          part_o,
+    const AttnSplitArgs a{q, k, v, k_cache, v_cache, pos, rope_cos, rope_sin, grp, max_len, splits, passes,
+                          direct_passes * kAsPass, scale, part_o,
                           reinterpret_cast<float2*>(part_o + (size_t)n_heads * splits * kAttnHD), counters, suh, o, xh};
     const dim3 grid((unsigned)splits, (unsigned)n_kv_heads, (unsigned)z);
     if (slots == 1) launch_attn_split<1>(grid, a, st);

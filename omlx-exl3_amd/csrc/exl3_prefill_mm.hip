@@ -402,7 +402,8 @@ static MmPlan mm_pair(int rows, int nsteps, int ti, int S) {
 // with x = w / 256, and f besides; S = 1 adds the epilogue, e (1 + 2.3 x), to each round, S > 1 the reduction launch: 2.13
 // us and S + 1 passes over an fp32 rows x n array at 2.4 TB/s up to 14 MB in all, 4.8 TB/s beyond.
 static double mm_us(const MmPlan& p, int rows, int n) {
-  static const double a[3] = {0.480, 0.683, 0.902}, b[3] = {-0.133, -0.291, -0.443}, c[3] = {0.211, 0.360, 0.497}, f[3] = {2.41, 3.23, 4.25}, e[3] = {3.19, 4.65, 6.02};
+  static const double a[3] = {0.480, 0.683, 0.902}, b[3] = {-0.133, -0.291, -0.443}, c[3] = {0.211, 0.360, 0.497};
+  static const double f[3] = {2.41, 3.23, 4.25}, e[3] = {3.19, 4.65, 6.02};   // (by tile height 128, 192, 256)
   const long groups = (long)p.tiles_m * ((n + kMmBN - 1) / kMmBN) * p.splits;
   const int i = p.ti - 2;
   auto round_us = [&](long w) {

@@ -5,15 +5,16 @@ EXL3Linear holds exactly the checkpoint tensors of one ExLlamaV3 linear (trellis
 the mul1 / mcg codebook marker, optional bias) as module buffers, so a strict `load_state_dict` fills it
 like any layer. Forward computes  y = had128( had128(x * suh) @ W_inner ) * svh  (+ bias):
 
-  rows <= MAX_GEMV_ROWS (decode, speculative verify): one GEMV launch that rotates the input (fp16 input;
-      other dtypes take a rotation launch first, and a primed rotated input is used as it is), reduces,
-      applies the output rotation, svh and the bias, and writes the caller's dtype (kernels.TrellisGemvPlan)
+  rows <= MAX_GEMV_ROWS (decode, speculative verify): one GEMV launch that rotates the input (fp16 or bf16),
+      reduces, applies the output rotation, svh and the bias, and writes the caller's dtype
+      (kernels.TrellisGemvPlan); fp32 input and several rows of a large layer take a rotation launch first
+      (kernels.ROTATE_IN_LAUNCH_LIMIT), and a primed rotated input is used as it is
   more rows (prefill, kernels.prefill_gemm): the input rotation, then for up to several hundred rows one launch
       that decodes each weight into the MFMA operands (exl3_prefill_rows; a second adds the k splits), else the
-      reference's sequence on hand-written kernels: W_inner^T reconstructed (bit-exact fp16) in column windows of bounded size, as the
-      reference decodes at most 16,384 columns at a time, each window multiplied by an MFMA GEMM whose
-      epilogue applies the output rotation, svh and bias (exl3_prefill_matmul; k split over workgroups for
-      few rows)
+      reference's sequence on hand-written kernels: W_inner^T reconstructed (bit-exact fp16) in column windows of
+      bounded size, as the reference decodes at most 16,384 columns at a time, each window multiplied by an MFMA
+      GEMM whose epilogue applies the output rotation, svh and bias (exl3_prefill_matmul_window; k split over
+      workgroups for few rows)
 
 EXL3SiblingGroup runs same-input siblings (q/k/v, gate/up) as one GEMV launch over their own trellis
 buffers when they share K and codebook; each member returns its slice of the output, held until every
@@ -385,7 +386,8 @@ class EXL3SiblingGroup:
 
     def gemv(self, x: torch.Tensor, out_dtype: torch.dtype) -> torch.Tensor:
         """All members' outputs, concatenated: (rows, sum(ns)) in out_dtype (rows <= MAX_GEMV_ROWS). The input
-        rotations run inside the GEMV launch for fp16 and bf16 input up to a measured amount, unless a rotated input was primed."""
+        rotations run inside the GEMV launch for fp16 and bf16 input up to a measured amount, unless a rotated
+        input was primed."""
         rows = x.numel() // self.k
         xh = self._primed.take(x)
         plan = self._plan(rows, out_dtype)
