@@ -284,7 +284,8 @@ class EXL3Linear(nn.Module):
     def _call_is_forward(self) -> bool:
         """Whether calling this module runs EXL3Linear.forward and nothing else (no hook, subclass, replaced or compiled
         forward, no output computed ahead), so that a caller may do forward's steps itself."""
-        return (type(self) is EXL3Linear and "forward" not in self.__dict__ and self._served.key is None
+        return (type(self) is EXL3Linear and EXL3Linear.forward is _FORWARD and "forward" not in self.__dict__
+                and self._served.key is None
                 and self._compiled_call_impl is None and not _has_any_global_hook()
                 and not (self._forward_hooks or self._forward_pre_hooks or self._backward_hooks or self._backward_pre_hooks))
 
@@ -322,6 +323,9 @@ class EXL3Linear(nn.Module):
             xh = rot(x.reshape(rows, self.in_features).contiguous(), self._suh2d).reshape(rows, self.in_features)
             y = self._prefill(xh, dtype, bias)
         return y.reshape(in_shape[:-1] + (self.out_features,))
+
+
+_FORWARD = EXL3Linear.forward
 
 
 class EXL3SiblingGroup:

@@ -415,7 +415,7 @@ def _fill(lin, seed):
                 else torch.randn(v.shape, generator=g).to(v.dtype)) for k, v in lin.state_dict().items()}
 
 
-@pytest.mark.parametrize("change", ["none", "load_state_dict", "data", "apply", "subclass", "forward", "hook", "pre_hook",
+@pytest.mark.parametrize("change", ["none", "load_state_dict", "data", "apply", "subclass", "forward", "class_forward", "hook", "pre_hook",
                                     "global_hook", "compiled", "served"])
 def test_group_prefill_follows_its_members(monkeypatch, change):
     """A grouped prefill gives what calling each member gives, whatever became of a member after grouping: scales loaded
@@ -447,6 +447,8 @@ def test_group_prefill_follows_its_members(monkeypatch, change):
         m._apply(lambda t: t.clone() * 2)
     elif change == "forward":
         m.forward = lambda x, f=m.forward: f(x) * 2
+    elif change == "class_forward":
+        monkeypatch.setattr(linear.EXL3Linear, "forward", lambda mod, x, f=linear.EXL3Linear.forward: f(mod, x) * 2)
     elif change == "hook":
         handle = m.register_forward_hook(lambda mod, a, y: seen.append(1) or y * 3)
     elif change == "pre_hook":
