@@ -19,6 +19,12 @@ def pk():
     return load_package()
 
 
+@pytest.fixture(autouse=True)
+def _no_kept_workspace(pk, monkeypatch):
+    """A call without a workspace takes the two launches, as when it is captured (eager it would use the thread's)."""
+    monkeypatch.setattr(pk.kernels._attn_scratch, "get", lambda *a: None)
+
+
 def _inputs(n_heads, n_kv, pos, max_len):
     g = torch.Generator(device="cuda").manual_seed(pos + n_heads + max_len)
 
